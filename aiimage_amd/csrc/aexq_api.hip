@@ -764,7 +764,7 @@ static aexq_status view_tensor(const aexq_tensor* t, const char* op, const char*
 // ---------------------------------------------------------------------------
 // strict plan
 // ---------------------------------------------------------------------------
-enum PlanKind : int { kPlanGeneric = 0, kPlanStream = 1, kPlanMfma = 2, kPlanGemm = 3 };
+enum PlanKind : int { kPlanGeneric = 0, kPlanStream = 1, kPlanMfma = 2, kPlanGemm = 3, kPlanWave = 4 };
 
 struct Plan {
   int kind = kPlanGeneric;
@@ -772,6 +772,8 @@ struct Plan {
   const QmvEntry* entry = nullptr;   // streaming kernel
   const QmmEntry* mentry = nullptr;  // MFMA kernel
   const QgemmEntry* gentry = nullptr;  // tiled GEMM (M > 32)
+  const QmmkEntry* kentry = nullptr;   // wave-split matmul
+  int kdepth = 0;                      // its LDS slots per wave
   int fmt = kQ8;
   int rows_per_tile = 0;
   QmvParams p{};
@@ -1096,8 +1098,45 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       plan->rms_prepass = rms_in;
     }
   };
-  if (M > 32 && gemm_shape_ok) try_gemm();
-  if (plan->kind != kPlanGemm && mfma_ok && size_ok) {
+  // launches with few output tiles: K split over a workgroup's waves
+  // (aexq_qmmk.hpp).  K % 128 == 0: M >= 2; up to 32 rows Q4 products stay
+  // exact and RMSNorm-in runs inside the kernel, above that Q4 weight tiles are
+  // fp16 and the norm is the row pre-pass, as in the tiled GEMM.  Any other K
+  // (rows past 8, or rows whose codes the streaming kernel cannot chunk): where
+  // only the generic kernel would be left (77 x 1008 x 1001: 5.7 us against
+  // 54.5); exact products.  The AEXQ_* switches that name another kernel's form
+  // keep that kernel.
+  auto try_wave = [&]() {
+    const bool rag = K % 128 != 0;
+    const int unit = fmt == kQ4 && w0->block == 32 ? 32 : 16;
+    if (argmax || !size_ok || K % unit != 0 || !(fmt == kQ8 || w0->block == 16 || w0->block == 32))
+      return;
+    if (rag ? swiglu || K % 64 == 0 || (M <= 8 && chunked) : M < 2 || (M > 32 && K < 512)) return;
+    for (const char* name : {"AEXQ_SPLITK", "AEXQ_QMM_NARROW", "AEXQ_QMM_BLOCKS_PER_CU", "AEXQ_QMMK_OFF"})
+      if (getenv(name)) return;
+    if (M > 32)
+      for (const char* name : {"AEXQ_QGEMM_OFF", "AEXQ_QGEMM_BM", "AEXQ_QGEMM_K64"})
+        if (getenv(name)) return;
+    const bool fused = rms_in && (rag || M <= 32) && getenv("AEXQ_RMS_PREPASS") == nullptr;
+    // (the kernel reads gamma[0 .. K) of fp16 rows)
+    if (fused ? !(rms_ok && x_ok) : !x_ok && !rms_in) return;
+    long long t16 = 0;
+    for (int i = 0; i < count; ++i)
+      t16 += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + 15) / 16 * w0->batch;
+    QmmkConfig kc{fmt, fmt == kQ8 ? 0 : w0->block, w0->scale_dtype == AEXQ_DTYPE_F16,
+                  !rag && M > 32 && fd, 1, 1, 8, swiglu, fused, rag};
+    if (!qmmk_pick(M, t16, swiglu, rag, &kc.mt, &kc.nt, &kc.waves)) return;
+    const char* env = getenv("AEXQ_QMMK_TILE");  // tuning: "mt:nt:waves"
+    if (env && sscanf(env, "%d:%d:%d", &kc.mt, &kc.nt, &kc.waves) != 3) return;
+    const QmmkEntry* e = qmmk_find(kc);
+    if (!e) return;
+    plan->kentry = e;
+    plan->kind = kPlanWave;
+    plan->rms_prepass = rms_in && !kc.rms;
+  };
+  try_wave();
+  if (plan->kind == kPlanGeneric && M > 32 && gemm_shape_ok) try_gemm();
+  if (plan->kind == kPlanGeneric && mfma_ok && size_ok) {
     const int mt = M <= 16 ? 1 : 2;
     // 256-wide K steps whose code fetches cover 128 contiguous bytes of 8 rows
     // per instruction, where K and the scale layout allow
@@ -1132,8 +1171,8 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
   // M = 9..32 where the MFMA block kernel does not apply (K a multiple of 64
   // but not of 128, Q4 scale groups of 64 or more): the tiled GEMM, its rows
   // past M masked, rather than the generic kernel
-  if (plan->kind != kPlanMfma && plan->kind != kPlanGemm && M > 8 && gemm_shape_ok) try_gemm();
-  if (plan->kind != kPlanMfma && plan->kind != kPlanGemm && chunked && group_ok && x_ok && m_ok && rms_ok && size_ok &&
+  if (plan->kind == kPlanGeneric && M > 8 && gemm_shape_ok) try_gemm();
+  if (plan->kind == kPlanGeneric && chunked && group_ok && x_ok && m_ok && rms_ok && size_ok &&
       chunks > 0) {
     const int mmax = M == 1 ? 1 : 8;
     int lpr = 0, cpl = 0;
@@ -1150,7 +1189,9 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       if (plan->fast) plan->kind = kPlanStream;
     }
   }
-  if (plan->kind == kPlanGemm) {
+  if (plan->kind == kPlanWave) {
+    plan->rows_per_tile = 16 * plan->kentry->cfg.nt;
+  } else if (plan->kind == kPlanGemm) {
     plan->rows_per_tile = qgemm_rows_per_tile(swiglu);
   } else if (plan->kind == kPlanMfma) {
     plan->rows_per_tile = plan->mentry->tn;
@@ -1239,8 +1280,8 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
   plan->x_rstride_in = xv.rstride;
   plan->x_bstride_in = xv.batch == 1 ? 0 : xv.bstride;
   plan->ysz = yv[0].dtype == AEXQ_DTYPE_F32 ? 4 : 2;
-  if (plan->kind == kPlanMfma || plan->kind == kPlanGemm) {
-    p.flags &= ~kFlagRms;  // normalised by the pre-pass
+  if (plan->kind == kPlanMfma || plan->kind == kPlanGemm || plan->kind == kPlanWave) {
+    p.flags &= ~kFlagRms;  // normalised by the pre-pass (or by an instantiation of its own)
     if (plan->rms_prepass) {
       // the scratch rows: [x batch][M][K] fp16 (pointer bound at launch)
       p.x_rstride = K;
@@ -1249,7 +1290,12 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
   }
   const int nw = swiglu ? 2 : 1;
   plan->sk_nw = nw;
-  if (plan->kind == kPlanGemm) {
+  if (plan->kind == kPlanWave) {
+    const int bm = 16 * plan->kentry->cfg.mt;
+    plan->mblock = bm;
+    plan->grid = (int)(((long long)tiles_total + 7) / 8 * 8 * ((M + bm - 1) / bm));
+    plan->kdepth = qmmk_depth(plan->kentry, K, (long long)tiles_total * ((M + bm - 1) / bm), ctx->cus);
+  } else if (plan->kind == kPlanGemm) {
     const int bm = plan->gentry->cfg.bm;
     const int mtiles = (M + bm - 1) / bm;
     plan->mblock = bm;
@@ -1368,6 +1414,11 @@ static aexq_status launch_mfma(aexq_ctx* ctx, Plan& plan, const char* op) {
     if (e != hipSuccess) return hip_fail(e, op, "rmsnorm pre-pass launch");
     for (int i = 0; i < p.nmat; ++i) p.mat[i].x = ctx->act_scratch;
   }
+  if (plan.kind == kPlanWave) {
+    hipError_t e = qmmk_launch(plan.kentry, p, plan.kdepth, ctx->stream);
+    if (e != hipSuccess) return hip_fail(e, op, "wave-split kernel launch");
+    return AEXQ_OK;
+  }
   // split K: the partial planes (sized for the largest row block) and, after
   // each kernel launch, the fix-up that sums them and runs the epilogue
   const bool split = plan.sk_chunks > 1;
@@ -1440,7 +1491,8 @@ static aexq_status launch_plan(aexq_ctx* ctx, Plan& plan, const char* op) {
     aexq_status st = gather_x(ctx, plan, op);
     if (st) return st;
   }
-  if (plan.kind == kPlanMfma || plan.kind == kPlanGemm) return launch_mfma(ctx, plan, op);
+  if (plan.kind == kPlanMfma || plan.kind == kPlanGemm || plan.kind == kPlanWave)
+    return launch_mfma(ctx, plan, op);
   hipError_t e = plan.fast ? qmv_launch(plan.entry, plan.p, plan.grid, ctx->stream)
                            : generic_launch(plan.fmt, plan.p, plan.grid, ctx->stream);
   if (e != hipSuccess) return hip_fail(e, op, "kernel launch");
@@ -1464,6 +1516,16 @@ extern "C" aexq_status aexq_plan_check(aexq_ctx* ctx, const aexq_weight* w, cons
                w->bits, plan.gentry->cfg.bm, (int)plan.gentry->cfg.pair,
                (int)plan.gentry->cfg.direct, (int)plan.gentry->cfg.fd, (int)plan.rms_prepass,
                plan.p.total_tiles, plan.grid, plan.sk_chunks, plan.gentry->cfg.k128 ? 128 : 64);
+    else if (plan.kind == kPlanWave)
+      // `splitk` counts the waves a tile's K is split over, inside one launch;
+      // `direct`: fragments straight from memory
+      snprintf(diag, diag_len,
+               "kernel=%s bits=%d mt=%d nt=%d bm=%d swiglu=%d wide=1 direct=1 fp16_dequant=%d "
+               "rms_prepass=%d tiles=%d grid=%d splitk=%d kstep=128",
+               plan.p.m <= 32 ? "qmmk" : "qgemmk", w->bits, plan.kentry->cfg.mt,
+               plan.kentry->cfg.nt, 16 * plan.kentry->cfg.mt, (int)plan.kentry->cfg.pair,
+               (int)plan.kentry->cfg.fd, (int)plan.rms_prepass, plan.p.total_tiles, plan.grid,
+               plan.kentry->cfg.waves);
     else if (plan.kind == kPlanMfma)
       snprintf(diag, diag_len, "kernel=qmm bits=%d mt=%d nt=%d swiglu=%d wide=%d rms_prepass=%d "
                "tiles=%d grid=%d mblock=%d splitk=%d",

@@ -68,6 +68,24 @@ __device__ __forceinline__ void q4_pairs(uint32_t w, uint32_t q[4]) {
   q[3] = as_u(__builtin_elementwise_fma(d, s_odd, b_odd));
 }
 
+// Eight offset-8 nibbles (n0 in bits 0-3) -> four fp16 pairs of the exact
+// codes n - 8 in element order: pair j = (n_2j, n_2j+1).  Byte j goes to both
+// halves (v_perm), the mask keeps n_2j low in half 0 and n_2j+1 at bits 4-7
+// of half 1; with the exponent pattern 0x6400 the halves are 1024 + n_2j and
+// 1024 + 16 n_2j+1, and one fma with (1, 1/16), (-1032, -72) gives both codes.
+__device__ __forceinline__ void q4_pairs_seq(uint32_t w, uint32_t q[4]) {
+  uint32_t E = 0x64006400u, m = 0x00F0000Fu;
+  __asm__("" : "+v"(E));
+  __asm__("" : "+s"(m));
+  const f16x2 mul = {(f16)1.0f, (f16)0.0625f};
+  const f16x2 add = {(f16)-1032.0f, (f16)-72.0f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t t = __builtin_amdgcn_perm(w, w, 0x0C000C00u | (j << 16) | j);
+    q[j] = as_u(__builtin_elementwise_fma(as_h2((t & m) | E), mul, add));
+  }
+}
+
 // Reorders 8 consecutive fp16 activations (a=(x0,x1) b=(x2,x3) c=(x4,x5)
 // d=(x6,x7)) into the (p, p+4) pairs that q4_pairs produces.
 __device__ __forceinline__ void q4_xpairs(uint32_t a, uint32_t b, uint32_t c, uint32_t d,

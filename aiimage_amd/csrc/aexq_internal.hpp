@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 namespace aexq {
 
 constexpr int kMaxGroup = 8;  // matrices per grouped launch
@@ -175,6 +177,35 @@ const QgemmEntry* qgemm_find(const QgemmConfig& cfg);
 int qgemm_rows_per_tile(bool pair);
 int qgemm_blocks_per_cu(const QgemmEntry* e);
 hipError_t qgemm_launch(const QgemmEntry* e, const QmvParams& p, hipStream_t stream);
+// Matmul with the K of a tile split over one workgroup's waves
+// (aexq_qmmk.hpp, instantiated in aexq_qmmk_*.hip): Q8, or Q4 with a scale
+// group of 16 or 32; tiles are 16 mt activation rows by 16 nt weight rows.
+struct QmmkConfig {
+  int fmt, g;      // g: Q4 scale group (16 or 32), 0 for Q8
+  bool sf16;       // fp16 (else fp32) scales
+  bool fd;         // Q4 weight tiles dequantised to fp16
+  int mt, nt, waves;
+  bool pair, rms;  // SwiGLU pair; RMSNorm-in inside the kernel
+  bool rag;        // K not a multiple of 128
+};
+typedef void (*QmmkFn)(const QmvParams, int, int);
+struct QmmkEntry {
+  QmmkConfig cfg;
+  QmmkFn fn;
+  int slot;  // LDS bytes of one slice
+  // devices on which fn may take more than 64 KB of dynamic LDS
+  mutable std::atomic<uint64_t> large_lds{0};
+};
+const QmmkEntry* qmmk_table_q8(int* count);
+const QmmkEntry* qmmk_table_q4(int* count);     // exact products
+const QmmkEntry* qmmk_table_q4_fd(int* count);  // fp16 weight tiles
+const QmmkEntry* qmmk_find(const QmmkConfig& cfg);
+// The tile and wave count for m rows by t16 16-row weight blocks (over every
+// matrix and copy); false: another kernel is the better one.
+bool qmmk_pick(int m, long long t16, bool pair, bool rag, int* mt, int* nt, int* waves);
+// LDS slots per wave of a launch of `wgs` workgroups on `cus` CUs
+int qmmk_depth(const QmmkEntry* e, int k, long long wgs, int cus);
+hipError_t qmmk_launch(const QmmkEntry* e, const QmvParams& p, int depth, hipStream_t stream);
 // RMSNorm of activation rows into fp16 rows (the M > 1 form of RMSNorm-in):
 // out[b][m][k] = fp16(x * rsqrt(max(mean(x^2) + eps, 1e-20)) * gamma[min(k, size-1)])
 hipError_t rmsnorm_rows_launch(const void* x, int x_f32, long long x_rstride, long long x_bstride,

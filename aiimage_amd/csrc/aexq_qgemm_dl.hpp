@@ -62,83 +62,16 @@
 // B[8 (l / 16) + j][l % 16], D[4 (l / 16) + r][l % 16], j < 8, r < 4.
 #pragma once
 
+#include "aexq_dma.hpp"
 #include "aexq_qmm.hpp"
 
 namespace aexq {
-
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) char gchar;  // global memory
-typedef __attribute__((address_space(1))) f32x4 gf32x4;
-typedef __attribute__((address_space(1))) u32x4 gu32x4;
-
-// LDS byte address of a generic pointer into LDS (the low half of the
-// generic address), wave-uniform.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p);
-}
-
-// One LDS-direct load: lane i's BYTES (16 or 4) at byte voff of resource r go
-// to LDS byte lds + BYTES * i; offsets past the resource's end write zeros.
-// Written as assembly so that the compiler does not see LDS stores in flight:
-// it would otherwise wait for every outstanding load before each LDS read.
-// The kernel orders them itself -- s_waitcnt vmcnt for its own loads, then a
-// barrier for the other waves' -- and the memory clobber keeps the compiler
-// from moving LDS accesses across a load.
-template <int BYTES>
-__device__ __forceinline__ void dma(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff) {
-  static_assert(BYTES == 16 || BYTES == 4, "dword or dwordx4");
-  if constexpr (BYTES == 16)
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds), "v"(voff), "s"(r)
-                 : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds), "v"(voff), "s"(r)
-                 : "memory", "m0");
-}
-
-// s_waitcnt vmcnt(N) with the other counters left alone (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | 0x70 | 0xF00 | ((N >> 4) << 14));
-}
-// s_waitcnt lgkmcnt(0).
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-// Workgroup barrier without the fence __syncthreads() adds (whose vmcnt(0)
-// would also wait for the LDS-direct loads of the steps ahead); the empty asm
-// statements keep the compiler from moving LDS accesses across it.
-__device__ __forceinline__ void bar() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // silu(g) = g / (1 + e^-g) with the division as a reciprocal (v_rcp_f32, 1 ulp)
 // times g: the SwiGLU epilogue of a tile forms it for every output, and the
 // IEEE division's expansion made up most of the epilogue's VALU work.
 __device__ __forceinline__ float silu_rcp(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-}
-
-// Eight offset-8 nibbles (n0 in bits 0-3) -> four fp16 pairs of the exact
-// codes n - 8 in element order: pair j = (n_2j, n_2j+1).  Byte j goes to both
-// halves (v_perm), the mask keeps n_2j low in half 0 and n_2j+1 at bits 4-7
-// of half 1; with the exponent pattern 0x6400 the halves are 1024 + n_2j and
-// 1024 + 16 n_2j+1, and one fma with (1, 1/16), (-1032, -72) gives both codes.
-__device__ __forceinline__ void q4_pairs_seq(uint32_t w, uint32_t q[4]) {
-  uint32_t E = 0x64006400u, m = 0x00F0000Fu;
-  __asm__("" : "+v"(E));
-  __asm__("" : "+s"(m));
-  const f16x2 mul = {(f16)1.0f, (f16)0.0625f};
-  const f16x2 add = {(f16)-1032.0f, (f16)-72.0f};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t t = __builtin_amdgcn_perm(w, w, 0x0C000C00u | (j << 16) | j);
-    q[j] = as_u(__builtin_elementwise_fma(as_h2((t & m) | E), mul, add));
-  }
 }
 
 template <int FMT, int BM, bool PAIR, bool SF16, int G, bool FD, int KS = 64>
@@ -634,20 +567,6 @@ struct QGemmDL {
     }
   }
 };
-
-// Waits until the loads of at most min(KMAX, ahead) steps (NL instructions
-// each) are outstanding, the older ones landed; `ahead` is wave-uniform.
-template <int NL, int KMAX>
-__device__ __forceinline__ void wait_steps(int ahead) {
-  if constexpr (KMAX > 0) {
-    if (ahead >= KMAX)
-      wait_vm<KMAX * NL>();
-    else
-      wait_steps<NL, KMAX - 1>(ahead);
-  } else {
-    wait_vm<0>();
-  }
-}
 
 // One step of the pipeline on LDS stage `cur` of an NST-stage ring (the next
 // step's stage `nxt`; the stage refilled with step st + NST is `cur` itself):
