@@ -1885,10 +1885,9 @@ static aexq_status attn_prepare(aexq_ctx* ctx, const char* op, int heads_q, int 
     return fail(AEXQ_ERR_UNSUPPORTED, op, "query heads per key head = %d (1, 2, 4 or 8)", group);
   if (length <= 0 || length > capacity)
     return fail(AEXQ_ERR_INVALID_ARGUMENT, op, "length=%d capacity=%d", length, capacity);
-  const int splits = attn_splits(length);
-  if (splits > attn_max_splits())
-    return fail(AEXQ_ERR_UNSUPPORTED, op, "length=%d needs %d splits (at most %d)", length,
-                splits, attn_max_splits());
+  if (length > attn_max_len())
+    return fail(AEXQ_ERR_UNSUPPORTED, op, "length=%d (at most %d)", length, attn_max_len());
+  const int splits = attn_splits(length, heads_kv, group);
   const long long need = (long long)heads_q * splits * attn_part_stride();
   HIP_TRY(op, hipSetDevice(ctx->device));
   aexq_status st = grow_scratch(ctx, (void**)&ctx->attn_part, &ctx->attn_cap,

@@ -10,6 +10,8 @@
 //                      softmax divided by max(sum, 1e-20), GQA key head = head / group)
 #include <math.h>
 
+#include <type_traits>
+
 #include "aexq_device.hpp"
 
 namespace aexq {
@@ -85,28 +87,34 @@ hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, v
 
 // ---------------------------------------------------------------------------
 // GQA decode attention in one launch.  Workgroup (kv head g, split c) covers
-// positions [64 c, 64 c + 64) of the `len` cached ones for the G = hq / hkv
-// query heads of g, so every cached K and V row is read once.  Every load of
-// the workgroup -- q, the RoPE tables and new row, then its K and V rows --
-// is issued before the first wait, and q (rotated here when RoPE is fused)
-// meets K after one barrier:
-//   scores   lanes 4i..4i+3 own position p0 + i, lane 4i + j the dims
-//            32 r + 8 j + [0, 8) for r < 4 (so one load instruction covers 64
-//            contiguous bytes of 16 rows), for all G heads (v_dot2 with fp32
-//            accumulation, quad reduction);
-//   softmax  max / sum per head over the split's positions (wave shuffles,
-//            then LDS across the 4 waves);
-//   P V      wave w owns positions p0 + 16 w + [0, 16), lane l dimensions
-//            2l and 2l + 1; the four waves' sums meet in LDS.
-// The split's (max, sum, acc[128]) per head goes to part[h][split].  The last
-// workgroup of kv head g to finish (a device-scope counter that the same
-// workgroup resets to 0, so the launch needs no clearing and replays inside a
-// graph) merges the splits of its G heads:
+// `per` positions (a multiple of 64) of the `len` cached ones for the G = hq /
+// hkv query heads of g, so every cached K and V row is read once.  Its four
+// waves run by themselves, 16 positions of each 64 per wave, with a running
+// maximum each and no barrier until the end:
+//   scores   lanes 4i..4i+3 own position i of the wave's 16, lane 4i + j the
+//            dims 32 r + 8 j + [0, 8) for r < 4 (so one load instruction covers
+//            64 contiguous bytes of 16 rows), for all G heads (v_dot2 with fp32
+//            accumulation, quad reduction by DPP);
+//   softmax  running max / sum per head over the wave's positions (DPP rows,
+//            then across rows);
+//   P V      lane group g4 = l / 16 owns positions 4 g4 + j, whose weights sit in
+//            its own DPP row (row_newbcast), lane l the dims 8 (l % 16) + [0, 8):
+//            four 16-byte loads cover the wave's 16 rows.
+// The next pass's K and V rows are requested before the current ones'
+// products (eight waves for splits of more than one four-wave pass), and q (rotated here when RoPE is fused) meets K after one barrier.
+// The waves' (max, sum, acc) meet in LDS; the split's go to part[h][split].
+// The last workgroup of kv head g to finish (a device-scope counter that the
+// same workgroup resets to 0, so the launch needs no clearing and replays
+// inside a graph) merges the splits of its G heads:
 //   M = max m_s, L = sum l_s e^(m_s - M), out = sum acc_s e^(m_s - M) / max(L, 1e-20).
+// That merge reads splits x G rows of 528 bytes through one CU, so a long cache
+// takes longer splits rather than more of them (attn_splits): with 64 positions
+// a split, 16 heads over 4 x 16384 positions took 22.6 us, half of them in the
+// merge, now 14.6 (32 MB: 5 us at the rate the shared cache level gives); up to
+// 64 positions there is one split and nothing to merge (7.4 -> 5.0 us).
 // head_dim == 128.
 // ---------------------------------------------------------------------------
 constexpr int kAttnDim = 128;
-constexpr int kAttnThreads = 256;
 
 // Device-coherent (agent scope) fp32 store / load: written through to, and
 // read from, the level all XCDs share.
@@ -116,22 +124,26 @@ __device__ __forceinline__ void store_coherent(float* p, float v) {
 __device__ __forceinline__ float load_coherent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-constexpr int kAttnPos = 64;         // positions per split
+constexpr int kAttnPos = 64;         // positions of a four-wave pass
 constexpr int kAttnStride = kAttnDim + 4;  // partial row: max, sum, 2 pad, acc[128] (16-byte aligned)
 constexpr int kCoherentAux = 16;     // buffer-load cache policy sc1: read at agent coherence
 // One counter per 256-byte line: atomics to one line are serialized where they
 // are performed (about 15 ns each), so the kv heads' counters do not share one.
 constexpr int kAttnCounterStride = 64;
-constexpr int kAttnMaxSplits = 512;  // combine staging in LDS
+constexpr int kAttnMaxSplits = 64;   // combine staging in LDS
+constexpr int kAttnMaxLen = 32768;   // positions a launch takes
 
-template <int G>
-__global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
+template <int G, int W>
+__global__ __launch_bounds__(64 * W) void attn_decode_kernel(
     const f16* q, const f16* kcache, const f16* vcache, int cap, int len, float scale,
     int splits, float* part, int* counters, f16* out, const f16* knew, const f16* vnew,
     f16* kcache_w, f16* vcache_w, const float* cosv, const float* sinv, const int* posp) {
   const int g = blockIdx.x, c = blockIdx.y;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   constexpr int half = kAttnDim / 2;
+  constexpr int T = 64 * W;     // threads
+  constexpr int P = 16 * W;     // positions of one pass
+  constexpr int RG = T / 32;    // row groups of the merge
   if (posp) {
     // decode position in device memory (a captured graph advances it): the
     // grid covers the cache capacity, the tables hold [cap][half] rows
@@ -140,15 +152,18 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     cosv += (long long)pp * half;
     sinv += (long long)pp * half;
   }
-  const int live_splits = (len + kAttnPos - 1) / kAttnPos;
-  const int p0 = c * kAttnPos;
-  const int pl = t >> 2, qq = t & 3;  // scores: position p0 + pl, dims 32 qq .. 32 qq + 31
+  // positions per split: the live length over the grid's splits
+  const int per = ((len + splits - 1) / splits + P - 1) / P * P;
+  const int live_splits = (len + per - 1) / per;
+  const int p0 = c * per, p1 = min(p0 + per, len);
+  const int pl = t >> 2, qq = t & 3;  // scores: position p0 + pl of a pass, dims 32 r + 8 qq ..
   const bool rope = knew != nullptr;
   const int pos = len - 1;             // the appended position when RoPE is fused
-  const bool has_new = rope && pos >= p0 && pos < p0 + kAttnPos;
+  const bool has_new = rope && pos >= p0 && pos < p0 + per;
   const long long head_off = (long long)g * cap * kAttnDim;
-  // P V sums: the four waves of a split, then the merge's eight row groups
-  __shared__ __align__(16) float pv[kAttnThreads / 32][G][kAttnDim];
+  // P V sums: the waves of a split, then the merge's row groups
+  __shared__ __align__(16) float pv[RG][G][kAttnDim];
+  __shared__ float wm[W][G], wl[W][G];
   __shared__ int last;
   if (c >= live_splits) {
     // a split past the live length (the grid was sized for the capacity):
@@ -161,7 +176,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     // 1. loads, all issued before the first wait; q and the new row first, so
     // that waiting for them leaves the K/V loads in flight.  Absent tables and
     // rows come through empty buffer resources (they read 0).
-    constexpr int QI = (G * half + kAttnThreads - 1) / kAttnThreads;  // (head, j) pairs per thread
+    constexpr int QI = (G * half + T - 1) / T;  // (head, j) pairs per thread
     float qa[QI], qb[QI], cs[QI], sn[QI];
     const __amdgpu_buffer_rsrc_t trs_c = __builtin_amdgcn_make_buffer_rsrc(
         (void*)cosv, (short)0, rope ? half * 4 : 0, kBufferRsrcWord3);
@@ -169,7 +184,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
         (void*)sinv, (short)0, rope ? half * 4 : 0, kBufferRsrcWord3);
 #pragma unroll
     for (int r = 0; r < QI; ++r) {
-      const int i = min(t + r * kAttnThreads, G * half - 1);
+      const int i = min(t + r * T, G * half - 1);
       const int h = i / half, j = i % half;
       const f16* qr = q + ((long long)g * G + h) * kAttnDim;
       qa[r] = (float)qr[j];
@@ -196,17 +211,25 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
         (void*)(kcache + head_off), (short)0, len * kAttnDim * 2, kBufferRsrcWord3);
     const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(vcache + head_off), (short)0, len * kAttnDim * 2, kBufferRsrcWord3);
-    u32x4 kreg[4];
+    // K: position q0 + pl of the P from q0, 64 bytes per lane; V: wave w's 16
+    // positions, lane group g4 rows 4 g4 + j, dims 8 (lane % 16) ..
+    const int g4 = lane >> 4, d8 = lane & 15;
+    struct Rows {
+      u32x4 k[4], v[4];
+    };
+    auto fetch = [&](int q0, Rows& r) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      kreg[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                              krs, (p0 + pl) * 256 + i * 64 + qq * 16, 0, 0));
-    // V rows: wave w owns positions p0 + 16 w + [0, 16), lane l dimensions 2l, 2l + 1
-    uint32_t vreg[16];
+      for (int i = 0; i < 4; ++i)
+        r.k[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               krs, (q0 + pl) * 256 + i * 64 + qq * 16, 0, 0));
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      vreg[i] = __builtin_amdgcn_raw_buffer_load_b32(
-          vrs, ((p0 + 16 * wave + i) * kAttnDim + 2 * lane) * 2, 0, 0);
+      for (int j = 0; j < 4; ++j)
+        r.v[j] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       vrs, (q0 + 16 * wave + 4 * g4 + j) * 256 + d8 * 16, 0, 0));
+    };
+    Rows cur, nxt;
+    fetch(p0, cur);
 
     // 2. q of the G heads (rotated and rounded to fp16 when RoPE is fused) and,
     // in the split that holds it, the appended K/V row
@@ -215,7 +238,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     __shared__ __align__(16) f16 vn[kAttnDim];
 #pragma unroll
     for (int r = 0; r < QI; ++r) {
-      const int i = t + r * kAttnThreads;
+      const int i = t + r * T;
       if (i < G * half) {
         const int h = i / half, j = i % half;
         qs[h][j] = rope ? (f16)(qa[r] * cs[r] - qb[r] * sn[r]) : (f16)qa[r];
@@ -240,129 +263,157 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
       vc[t + half] = v1;
     }
     __syncthreads();
-    if (has_new) {
-      // the cache row at `pos` was loaded before it was written: take the new one
-      if (p0 + pl == pos) {
+    // 3. the split's positions, P at a time; every wave keeps its own running
+    // maximum, sum and accumulators
+    float mx[G], sm[G], ac[G][8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) kreg[i] = *(const u32x4*)&kn[i * 32 + qq * 8];
+    for (int h = 0; h < G; ++h) {
+      mx[h] = -INFINITY;
+      sm[h] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ac[h][e] = 0.0f;
+    }
+    auto take = [&](int q0, Rows& r, auto first) {
+      constexpr bool FIRST = decltype(first)::value;
+      if (has_new && q0 + P > pos) {
+        // the cache row at `pos` was loaded before it was written: take the new one
+        if (q0 + pl == pos) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r.k[i] = *(const u32x4*)&kn[i * 32 + qq * 8];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (q0 + 16 * wave + 4 * g4 + j == pos) r.v[j] = *(const u32x4*)&vn[8 * d8];
       }
+      if (q0 + 16 * wave < p1) {  // the wave's first position is live
+        const bool live = q0 + pl < len;
+        float sc[G];
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (p0 + 16 * wave + i == pos) vreg[i] = *(const uint32_t*)&vn[2 * lane];
-    }
-
-    // 3. scores of position p0 + pl for every head (quad sums by DPP)
-    const bool live = p0 + pl < len;
-    float sc[G];
+        for (int h = 0; h < G; ++h) {
+          float acc = 0.0f;
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float acc = 0.0f;
+          for (int i = 0; i < 4; ++i) {
+            const u32x4 qw = *(const u32x4*)&qs[h][i * 32 + qq * 8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const u32x4 qw = *(const u32x4*)&qs[h][i * 32 + qq * 8];
+            for (int e = 0; e < 4; ++e) acc = dot2(r.k[i][e], qw[e], acc);
+          }
+          sc[h] = acc;
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = dot2(kreg[i][e], qw[e], acc);
-      }
-      sc[h] = acc;
-    }
+        for (int h = 0; h < G; ++h) sc[h] += dpp<0xB1>(sc[h]);  // quad_perm [1,0,3,2]
 #pragma unroll
-    for (int h = 0; h < G; ++h) sc[h] += dpp<0xB1>(sc[h]);  // quad_perm [1,0,3,2]
+        for (int h = 0; h < G; ++h) {
+          sc[h] += dpp<0x4E>(sc[h]);  // quad_perm [2,3,0,1]
+          sc[h] = live ? sc[h] * scale : -INFINITY;
+        }
+        float ex[G], mx0[G];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      sc[h] += dpp<0x4E>(sc[h]);  // quad_perm [2,3,0,1]
-      sc[h] = live ? sc[h] * scale : -INFINITY;
-    }
-
-    // 4. softmax statistics of the split per head: the 16 positions of a wave
-    // reduce within DPP rows (row_ror 4, 8), then across rows with the lane
-    // shuffles of all heads issued together; the 4 waves meet in LDS
-    __shared__ float red[kAttnThreads / 64][G];
-    __shared__ float es[G][kAttnPos];
-    float mx[G], rr[G];
+        for (int h = 0; h < G; ++h) {
+          // maximum over the wave's 16 positions: within DPP rows, then across
+          float m = fmaxf(sc[h], dpp<0x124>(sc[h]));
+          m = fmaxf(m, dpp<0x128>(m));
+          m = fmaxf(m, dpp_rows<0x142, 0xA>(m, m));
+          m = fmaxf(m, dpp_rows<0x143, 0xC>(m, m));
+          mx0[h] = mx[h];
+          mx[h] = fmaxf(mx0[h], lane_value(m, 63));
+          // (scores that are all -inf so far weigh 0, not NaN)
+          const float base = mx[h] == -INFINITY ? 0.0f : mx[h];
+          ex[h] = live ? __expf(sc[h] - base) : 0.0f;
+          float s = ex[h] + dpp<0x124>(ex[h]);
+          s += dpp<0x128>(s);
+          // what came before, on the new maximum (nothing in the first pass)
+          const float corr = FIRST ? 0.0f : __expf(mx0[h] - base);
+          sm[h] = fmaf(sm[h], corr, s);  // of the lane's own row until the end
+          if constexpr (!FIRST) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      rr[h] = fmaxf(sc[h], dpp<0x124>(sc[h]));
-      rr[h] = fmaxf(rr[h], dpp<0x128>(rr[h]));
-    }
+            for (int e = 0; e < 8; ++e) ac[h][e] *= corr;
+          }
+        }
+        // rows past the end read 0 and weigh 0
+        auto weigh = [&](int j, float w, int h) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) rr[h] = fmaxf(rr[h], __shfl_xor(rr[h], 16, 64));
+          for (int e = 0; e < 4; ++e) {
+            const f16x2 vv = as_h2(r.v[j][e]);
+            ac[h][2 * e] = fmaf(w, (float)vv[0], ac[h][2 * e]);
+            ac[h][2 * e + 1] = fmaf(w, (float)vv[1], ac[h][2 * e + 1]);
+          }
+        };
 #pragma unroll
-    for (int h = 0; h < G; ++h) rr[h] = fmaxf(rr[h], __shfl_xor(rr[h], 32, 64));
-    if (lane == 0) {
-#pragma unroll
-      for (int h = 0; h < G; ++h) red[wave][h] = rr[h];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float m = red[0][h];
-#pragma unroll
-      for (int w = 1; w < kAttnThreads / 64; ++w) m = fmaxf(m, red[w][h]);
-      mx[h] = m;  // finite: every split holds at least one live position
-    }
-    __syncthreads();
-    float ex[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      ex[h] = live ? __expf(sc[h] - mx[h]) : 0.0f;
-      rr[h] = ex[h] + dpp<0x124>(ex[h]);
-      rr[h] += dpp<0x128>(rr[h]);
-    }
-#pragma unroll
-    for (int h = 0; h < G; ++h) rr[h] += __shfl_xor(rr[h], 16, 64);
-#pragma unroll
-    for (int h = 0; h < G; ++h) rr[h] += __shfl_xor(rr[h], 32, 64);
-    if (qq == 0) {
-#pragma unroll
-      for (int h = 0; h < G; ++h) es[h][pl] = ex[h];
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int h = 0; h < G; ++h) red[wave][h] = rr[h];
-    }
-    __syncthreads();
-    float sm[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float s = 0.0f;
-#pragma unroll
-      for (int w = 0; w < kAttnThreads / 64; ++w) s += red[w][h];
-      sm[h] = s;
-    }
-
-    // 5. P V: wave w, dimensions 2 lane and 2 lane + 1 over its 16 positions;
-    // the four waves' sums meet in LDS
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float e = es[h][16 * wave + i];
-        const f16x2 vv = as_h2(vreg[i]);
-        a0 = fmaf(e, (float)vv[0], a0);
-        a1 = fmaf(e, (float)vv[1], a1);
-      }
-      pv[wave][h][2 * lane] = a0;
-      pv[wave][h][2 * lane + 1] = a1;
-    }
-    __syncthreads();
-    const int d = t & (kAttnDim - 1), vh = t >> 7;
-    if (vh == 0) {
-#pragma unroll
-      for (int h = 0; h < G; ++h) {
-        float a = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kAttnThreads / 64; ++w) a += pv[w][h][d];
-        float* o = part + ((long long)(g * G + h) * splits + c) * kAttnStride;
-        store_coherent(o + 4 + d, a);
-        if (d == 0) {
-          store_coherent(o, mx[h]);
-          store_coherent(o + 1, sm[h]);
+        for (int h = 0; h < G; ++h) {
+          weigh(0, dpp<0x150>(ex[h]), h);  // row_newbcast: lane 4 j of the lane's row
+          weigh(1, dpp<0x154>(ex[h]), h);
+          weigh(2, dpp<0x158>(ex[h]), h);
+          weigh(3, dpp<0x15C>(ex[h]), h);
         }
       }
+    };
+    // a split of one pass, with no rows of a next one on the way
+    if (per == P) {
+      take(p0, cur, std::true_type{});
+    } else {
+      for (int q0 = p0; q0 < p1; q0 += P) {
+        fetch(q0 + P < p1 ? q0 + P : len, nxt);  // past the last row: no traffic
+        __builtin_amdgcn_sched_barrier(0);
+        take(q0, cur, std::false_type{});
+        cur = nxt;
+      }
     }
 
-    // 6. the last split of kv head g merges all of them.  Partials travel
+    // 4. over the four rows of the wave, then over the waves in LDS
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      float l = sm[h];
+      l += dpp_rows<0x142, 0xA>(0.0f, l);
+      l += dpp_rows<0x143, 0xC>(0.0f, l);
+      if (lane == 63) {
+        wm[wave][h] = mx[h];
+        wl[wave][h] = l;
+      }
+      // two sums per swap: halves of the wave, then rows of the halves; row
+      // r ends with dims 8 d8 + (0, 2, 1, 3)[r] and that + 4
+      float s2[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto r = __builtin_amdgcn_permlane32_swap(f32_bits(ac[h][2 * e]),
+                                                        f32_bits(ac[h][2 * e + 1]), false, false);
+        s2[e] = as_f32(r[0]) + as_f32(r[1]);
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const auto r = __builtin_amdgcn_permlane16_swap(f32_bits(s2[2 * e]), f32_bits(s2[2 * e + 1]),
+                                                        false, false);
+        pv[wave][h][8 * d8 + 4 * e + (g4 >> 1) + 2 * (g4 & 1)] = as_f32(r[0]) + as_f32(r[1]);
+      }
+    }
+    __syncthreads();
+    for (int i = t; i < G * kAttnDim; i += T) {
+      const int h = i / kAttnDim, d = i % kAttnDim;
+      float m = wm[0][h];
+#pragma unroll
+      for (int w = 1; w < W; ++w) m = fmaxf(m, wm[w][h]);
+      const float base = m == -INFINITY ? 0.0f : m;
+      float a = 0.0f, l = 0.0f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float f = __expf(wm[w][h] - base);  // a wave with no live position: 0
+        a = fmaf(pv[w][h][d], f, a);
+        l = fmaf(wl[w][h], f, l);
+      }
+      if (splits == 1) {  // nothing to merge
+        const float f = __expf(m - m);  // NaN where every score is -inf, as in the merge
+        out[((long long)g * G + h) * kAttnDim + d] = (f16)(a * f / fmaxf(l * f, 1e-20f));
+        continue;
+      }
+      float* o = part + ((long long)(g * G + h) * splits + c) * kAttnStride;
+      store_coherent(o + 4 + d, a);
+      if (d == 0) {
+        store_coherent(o, m);
+        store_coherent(o + 1, l);
+      }
+    }
+    if (splits == 1) return;
+
+    // 5. the last split of kv head g merges all of them.  Partials travel
     // through device-coherent stores and loads (they bypass the per-XCD L2
     // that plain accesses would leave stale), ordered by waiting for the
     // stores before the counter increment.
@@ -375,7 +426,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
   // Loads of the merge: the split statistics (row t of the G * splits rows
   // (head, split) in registers), then the first chunk of accumulator rows, all
   // in flight together.  Thread (rg = t / 32, dq = t % 32) reads dims 4 dq ..
-  // 4 dq + 3 of splits rg + 8 j of every head; splits past the last live one
+  // 4 dq + 3 of splits rg + RG j of every head; splits past the last live one
   // are sent out of the buffer range, which reads 0.  Rows keep the grid's
   // pitch (`splits`); only the first live_splits of each head hold partials
   // of this launch.
@@ -387,7 +438,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
   const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
       (void*)pg, (short)0, rows * kAttnStride * 4, kBufferRsrcWord3);
   constexpr int JJ = 16 / G;  // accumulator rows per head and thread in one chunk
-  constexpr int kChunk = 8 * JJ;
+  constexpr int kChunk = RG * JJ;
   const int dq = t & 31, rg = t >> 5;
   const float m0 = as_f32(__builtin_amdgcn_raw_buffer_load_b32(prs, t * kAttnStride * 4, 0, kCoherentAux));
   const float l0 = as_f32(__builtin_amdgcn_raw_buffer_load_b32(prs, (t * kAttnStride + 1) * 4, 0, kCoherentAux));
@@ -397,7 +448,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     for (int h = 0; h < G; ++h)
 #pragma unroll
       for (int j = 0; j < JJ; ++j) {
-        const int s2 = s0 + rg + 8 * j;
+        const int s2 = s0 + rg + RG * j;
         const int off = s2 < nsp ? ((h * splits + s2) * kAttnStride + 4 + 4 * dq) * 4 : 0x7FFFFFF0;
         av[h][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(prs, off, 0, kCoherentAux));
       }
@@ -408,7 +459,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     cm[t] = ok ? m0 : -INFINITY;
     cl[t] = ok ? l0 : 0.0f;
   }
-  for (int i = t + kAttnThreads; i < rows; i += kAttnThreads) {
+  for (int i = t + T; i < rows; i += T) {
     const bool ok = i % splits < nsp;
     cm[i] = ok ? as_f32(__builtin_amdgcn_raw_buffer_load_b32(prs, i * kAttnStride * 4, 0, kCoherentAux))
                : -INFINITY;
@@ -418,7 +469,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
   __syncthreads();
   // per head: M = max m_s (each wave reduces the heads h == wave mod 4)
   __shared__ float hm[G], hl[G];
-  for (int h = wave; h < G; h += kAttnThreads / 64) {
+  for (int h = wave; h < G; h += W) {
     float m = -INFINITY;
     for (int s2 = lane; s2 < nsp; s2 += 64) m = fmaxf(m, cm[h * splits + s2]);
     m = wave_max(m);
@@ -445,7 +496,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     for (int h = 0; h < G; ++h)
 #pragma unroll
       for (int j = 0; j < JJ; ++j) {
-        const int s2 = min(s0 + rg + 8 * j, nsp - 1);  // rows past the end loaded 0
+        const int s2 = min(s0 + rg + RG * j, nsp - 1);  // rows past the end loaded 0
         const float w = cm[h * splits + s2];
 #pragma unroll
         for (int e = 0; e < 4; ++e) ac[h][e] = fmaf(as_f32(av[h][j][e]), w, ac[h][e]);
@@ -454,18 +505,18 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
     if (s0 >= nsp) break;
     issue(s0);
   }
-  // the eight row groups' sums meet in LDS
+  // the row groups' sums meet in LDS
 #pragma unroll
   for (int h = 0; h < G; ++h) {
     const f32x4 v = {ac[h][0], ac[h][1], ac[h][2], ac[h][3]};
     *(f32x4*)&pv[rg][h][4 * dq] = v;
   }
   __syncthreads();
-  for (int i = t; i < G * kAttnDim; i += kAttnThreads) {
+  for (int i = t; i < G * kAttnDim; i += T) {
     const int h = i / kAttnDim, dd = i % kAttnDim;
     float a = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kAttnThreads / 32; ++w) a += pv[w][h][dd];
+    for (int w = 0; w < RG; ++w) a += pv[w][h][dd];
     out[((long long)g * G + h) * kAttnDim + dd] = (f16)(a / fmaxf(hl[h], 1e-20f));
   }
   if (t == 0) counters[g * kAttnCounterStride] = 0;  // ready for the next launch
@@ -492,8 +543,18 @@ hipError_t decode_advance_launch(int* position, int* token, const int* argmax, i
   return hipGetLastError();
 }
 
-int attn_splits(int len) { return (len + kAttnPos - 1) / kAttnPos; }
-int attn_max_splits() { return kAttnMaxSplits; }
+// Splits per kv head of a launch over len positions: 64 positions each as long
+// as that keeps the merge short, then longer ones.  Measured (us, heads_q /
+// heads_kv, splits at most 32, 64, 128; with 64 positions a split always):
+// 16/4 at 4096 8.9, 9.5, 9.6 (9.3), at 16384 16.5, 14.6, 18.0 (22.6); 8/1 at
+// 4096 12.1, 14.4, 14.5 (14.5), at 16384 23.0, 18.8, 19.3 (29.1); 32/8 at 8192
+// 14.2, 16.1, 19.0 (18.4); 4/4, whose merge is a quarter, at 4096 7.1, 6.8.
+int attn_splits(int len, int heads_kv, int group) {
+  const int most = len <= 4096 ? (group >= 4 ? 32 : 64) : (heads_kv >= 8 ? 32 : 64);
+  const int s = (len + kAttnPos - 1) / kAttnPos;
+  return s < most ? s : most;
+}
+int attn_max_len() { return kAttnMaxLen; }
 int attn_part_stride() { return kAttnStride; }
 int attn_counter_stride() { return kAttnCounterStride; }
 
@@ -505,14 +566,18 @@ hipError_t attn_decode_launch(const void* q, const void* kcache, const void* vca
   // a device-side position: the grid covers the capacity, the kernel reads
   // the live length
   if (posp) len = cap;
-  const int splits = attn_splits(len);
-  if (splits > kAttnMaxSplits) return hipErrorInvalidValue;
+  const int splits = attn_splits(len, hkv, group);
+  if (len > kAttnMaxLen || splits < 1 || splits > kAttnMaxSplits) return hipErrorInvalidValue;
   const dim3 grid(hkv, splits);
-#define AEXQ_ATTN(G)                                                                             \
-  hipLaunchKernelGGL(attn_decode_kernel<G>, grid, dim3(kAttnThreads), 0, stream, (const f16*)q, \
+  // longer splits take eight waves: twice the rows on the way to each CU
+  const bool wide = len > kAttnPos * splits;
+#define AEXQ_ATTN_W(G, W)                                                                        \
+  hipLaunchKernelGGL((attn_decode_kernel<G, W>), grid, dim3(64 * W), 0, stream, (const f16*)q,  \
                      (const f16*)kcache, (const f16*)vcache, cap, len, scale, splits, part,      \
                      counters, (f16*)out, (const f16*)knew, (const f16*)vnew, (f16*)kcache,      \
                      (f16*)vcache, cosv, sinv, (const int*)posp)
+#define AEXQ_ATTN(G) \
+  if (wide) AEXQ_ATTN_W(G, 8); else AEXQ_ATTN_W(G, 4)
   switch (group) {
     case 1: AEXQ_ATTN(1); break;
     case 2: AEXQ_ATTN(2); break;
@@ -521,6 +586,7 @@ hipError_t attn_decode_launch(const void* q, const void* kcache, const void* vca
     default: return hipErrorInvalidValue;
   }
 #undef AEXQ_ATTN
+#undef AEXQ_ATTN_W
   return hipGetLastError();
 }
 
