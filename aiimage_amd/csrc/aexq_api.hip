@@ -1091,6 +1091,25 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       const bool k128 = fmt == kQ4 && fd && bm == 64 && K % 128 == 0 &&
                         getenv("AEXQ_QGEMM_K64") == nullptr;
       gc = QgemmConfig{fmt, bm, swiglu, sf16, g16, true, fd, k128};
+      // eight waves on a tile, two along its rows, where the switches of the
+      // four-wave forms are off
+      long long tiles = 0;  // of 128 x 128
+      for (int i = 0; i < count; ++i)
+        tiles += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + (swiglu ? 63 : 127)) /
+                 (swiglu ? 64 : 128) * w0->batch;
+      tiles *= (M + 127) / 128;
+      if (M > 64 && (fmt == kQ8 || fd) && !benv && !getenv("AEXQ_QGEMM_K64") && !getenv("AEXQ_SPLITK")) {
+        // From 96 tiles to one (Q4, whose codes each row half of the tile expands
+        // again) or two per CU (Q8), all resident at once and unsplit: the
+        // four-wave tile leaves one wave a SIMD there, or splits K and pays the
+        // partial planes (us, 1000 x 4096 x 4096: Q8 43 against 66, Q4-g16 47
+        // against 63; 512 x 8192 x 2048 Q8 26 against 30).  Past that its two
+        // workgroups a CU do as well with less expansion (2048 x 4096 x 1024 Q4 30
+        // against 37), and tiles of 256 weight rows were no faster (2048 x 8192
+        // pairs x 2048 Q8: 159 against 154 with half the bytes per product).
+        if (tiles >= 96 && tiles <= (fmt == kQ8 ? 2 : 1) * ctx->cus && (fmt == kQ8 || K % 128 == 0))
+          gc = QgemmConfig{fmt, 128, swiglu, sf16, g16, true, fd, fmt == kQ4, 2};
+      }
     }
     plan->gentry = qgemm_find(gc);
     if (plan->gentry) {
@@ -1125,7 +1144,7 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       t16 += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + 15) / 16 * w0->batch;
     QmmkConfig kc{fmt, fmt == kQ8 ? 0 : w0->block, w0->scale_dtype == AEXQ_DTYPE_F16,
                   !rag && M > 32 && fd, 1, 1, 8, swiglu, fused, rag};
-    if (!qmmk_pick(M, t16, swiglu, rag, &kc.mt, &kc.nt, &kc.waves)) return;
+    if (!qmmk_pick(M, t16, fmt == kQ8, swiglu, rag, &kc.mt, &kc.nt, &kc.waves)) return;
     const char* env = getenv("AEXQ_QMMK_TILE");  // tuning: "mt:nt:waves"
     if (env && sscanf(env, "%d:%d:%d", &kc.mt, &kc.nt, &kc.waves) != 3) return;
     const QmmkEntry* e = qmmk_find(kc);
@@ -1315,10 +1334,11 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
     // and 512 measured fastest at 4 to 8, slower at 14 to 28)
     const int kstep = plan->gentry->cfg.k128 ? 128 : 64;  // K per step of the kernel
     if (plan->gentry->cfg.k128) step_us *= 2.0;
-    pick_split((long long)tiles_total * mtiles, K / kstep, slots, step_us, wg_us,
-               plan->gentry->cfg.direct ? 8 : 1 << 30,
-               (double)M * nw * tiles_total * plan->rows_per_tile * 4.0,
-               &plan->sk_chunks, &plan->sk_cs);
+    if (plan->gentry->cfg.wm == 1)  // (the eight-wave tiles come with enough of them)
+      pick_split((long long)tiles_total * mtiles, K / kstep, slots, step_us, wg_us,
+                 plan->gentry->cfg.direct ? 8 : 1 << 30,
+                 (double)M * nw * tiles_total * plan->rows_per_tile * 4.0,
+                 &plan->sk_chunks, &plan->sk_cs);
     plan->grid = (int)(((long long)tiles_total + 7) / 8 * 8 * mtiles * plan->sk_chunks);
   } else if (plan->kind == kPlanMfma) {
     int per_cu = qmm_blocks_per_cu(plan->mentry);

@@ -166,7 +166,8 @@ struct QgemmConfig {
   bool g16;    // Q4 with one scale per 16 codes
   bool direct; // LDS-direct pipeline (Q8; Q4 split scales in groups of 16 or 32)
   bool fd;     // Q4 weight tiles dequantised to fp16 (fp16(q * s)) for the MFMA
-  bool k128;   // fd at 64-row tiles: 128-wide K steps (K a multiple of 128)
+  bool k128;   // fd: 128-wide K steps (K a multiple of 128)
+  int wm = 1;    // waves along the activation rows, by four along the weight rows
 };
 typedef void (*QgemmFn)(const QmvParams, int);
 struct QgemmEntry {
@@ -174,6 +175,7 @@ struct QgemmEntry {
   QgemmFn fn;
 };
 const QgemmEntry* qgemm_find(const QgemmConfig& cfg);
+const QgemmEntry* qgemm_table_wide(int* count);  // the eight-wave entries (aexq_qgemm_wide.hip)
 int qgemm_rows_per_tile(bool pair);
 int qgemm_blocks_per_cu(const QgemmEntry* e);
 hipError_t qgemm_launch(const QgemmEntry* e, const QmvParams& p, hipStream_t stream);
@@ -202,7 +204,7 @@ const QmmkEntry* qmmk_table_q4_fd(int* count);  // fp16 weight tiles
 const QmmkEntry* qmmk_find(const QmmkConfig& cfg);
 // The tile and wave count for m rows by t16 16-row weight blocks (over every
 // matrix and copy); false: another kernel is the better one.
-bool qmmk_pick(int m, long long t16, bool pair, bool rag, int* mt, int* nt, int* waves);
+bool qmmk_pick(int m, long long t16, bool q8, bool pair, bool rag, int* mt, int* nt, int* waves);
 // LDS slots per wave of a launch of `wgs` workgroups on `cus` CUs
 int qmmk_depth(const QmmkEntry* e, int k, long long wgs, int cus);
 hipError_t qmmk_launch(const QmmkEntry* e, const QmvParams& p, int depth, hipStream_t stream);

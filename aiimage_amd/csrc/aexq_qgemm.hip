@@ -46,11 +46,16 @@ static const QgemmEntry kTableG[] = {QGE(false, true), QGE(false, false), QGE(tr
 static constexpr int kCountG = (int)(sizeof(kTableG) / sizeof(kTableG[0]));
 
 const QgemmEntry* qgemm_find(const QgemmConfig& c) {
-  for (int i = 0; i < kCountG; ++i) {
-    const QgemmConfig& q = kTableG[i].cfg;
+  int nw = 0;
+  const QgemmEntry* tw = qgemm_table_wide(&nw);
+  const QgemmEntry* t = c.wm == 1 ? kTableG : tw;
+  const int n = c.wm == 1 ? kCountG : nw;
+  for (int i = 0; i < n; ++i) {
+    const QgemmConfig& q = t[i].cfg;
     if (q.fmt == c.fmt && q.bm == c.bm && q.pair == c.pair && q.sf16 == c.sf16 &&
-        q.g16 == c.g16 && q.direct == c.direct && q.fd == c.fd && q.k128 == c.k128)
-      return &kTableG[i];
+        q.g16 == c.g16 && q.direct == c.direct && q.fd == c.fd && q.k128 == c.k128 &&
+        q.wm == c.wm)
+      return &t[i];
   }
   return nullptr;
 }
@@ -60,7 +65,7 @@ int qgemm_rows_per_tile(bool pair) { return pair ? 64 : 128; }
 int qgemm_blocks_per_cu(const QgemmEntry* e) {
   static int cache[kCountG] = {0};
   const int idx = (int)(e - kTableG);
-  if (idx < 0 || idx >= kCountG) return 1;
+  if (idx < 0 || idx >= kCountG) return 1;  // the eight-wave tiles fill a CU's LDS
   if (cache[idx] == 0) {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, e->fn, kThreads, 0) != hipSuccess || n < 1)
@@ -76,7 +81,7 @@ hipError_t qgemm_launch(const QgemmEntry* e, const QmvParams& p, hipStream_t str
   const long long groups = (p.total_tiles + 7) / 8;
   const long long grid = groups * 8 * mtiles * (p.sk_chunks > 1 ? p.sk_chunks : 1);
   if (grid <= 0 || grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(e->fn, dim3((unsigned)grid), dim3(kThreads), 0, stream, p, mtiles);
+  hipLaunchKernelGGL(e->fn, dim3((unsigned)grid), dim3(kThreads * e->cfg.wm), 0, stream, p, mtiles);
   return hipGetLastError();
 }
 

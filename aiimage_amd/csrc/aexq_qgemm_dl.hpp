@@ -49,7 +49,10 @@
 //
 // Waves: 1 x 4, each every activation row of the tile by 32 weight rows, so
 // a code fragment is expanded to fp16 once per workgroup (a 2 x 2 layout
-// expands every B block in two waves: Q4 at M = 512 measured 7% slower).
+// expands every B block in two waves: Q4 at M = 512 measured 7% slower).  For
+// launches of about one or two tiles per CU, 2 x 4 (WM = 2): eight waves a tile
+// hide what two workgroups per CU hide elsewhere, for a second expansion of the
+// codes (1000 x 4096 x 4096, us: Q8 66 -> 43, Q4 in groups of 16 63 -> 47).
 // Inside a step the barrier sits between the two K halves: the first half's
 // MFMAs cover the second half's fragment reads and the barrier wait, the
 // second half's MFMAs cover the next step's first fragment reads.
@@ -74,7 +77,7 @@ __device__ __forceinline__ float silu_rcp(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
 }
 
-template <int FMT, int BM, bool PAIR, bool SF16, int G, bool FD, int KS = 64>
+template <int FMT, int BM, bool PAIR, bool SF16, int G, bool FD, int KS = 64, int WM_ = 1>
 struct QGemmDL {
   static_assert(FMT == kQ8 ? G == 0 : (G == 16 || G == 32),
                 "Q8 (row scales) or Q4 in groups of 16 or 32");
@@ -82,13 +85,17 @@ struct QGemmDL {
   static_assert(BM == 64 || BM == 128, "64- or 128-row activation tiles");
   static_assert(KS == 64 || (KS == 128 && FD), "128-wide K steps are a form of Q4 fp16 tiles");
   static constexpr int BN = 128;                  // weight rows of a tile
+  static constexpr int WM = WM_;                  // waves along the activation rows
+  static constexpr int WAVES = 4 * WM;            // ... by four along the weight rows
+  static constexpr int THREADS = 64 * WAVES;
+  static constexpr int HB = BN / 2;               // weight rows of each half of a pair
   static constexpr int BK = KS;                   // K per step
   static constexpr int NE = BK / 32;              // MFMA K extents per step
   static constexpr int RA = 2 * BK;               // activation bytes per row and step
   static constexpr int NOUT = PAIR ? BN / 2 : BN;  // output columns of a tile
-  static constexpr int WR = BN / 4;               // weight rows per wave (32)
-  static constexpr int TN = WR / 16;              // 16-row B blocks per wave (2)
-  static constexpr int TM = BM / 16;              // 16-row A blocks per wave (every row)
+  static constexpr int WR = BN / 4;               // weight rows per wave
+  static constexpr int TN = WR / 16;              // 16-row B blocks per wave
+  static constexpr int TM = BM / 16 / WM;         // 16-row A blocks per wave
   static constexpr int CP = FMT == kQ8 ? 64 : BK / 2;  // code bytes per row and step
   // codes read as Q8's: a lane's 16 bytes of a 64-byte row step (Q8, Q4 at KS 128)
   static constexpr bool C16 = CP == 64;
@@ -97,20 +104,21 @@ struct QGemmDL {
   static constexpr int SPR = FMT == kQ8 ? 0 : BK / G;    // Q4 scales per row and step
   static constexpr int SB = SF16 ? 2 : 4;                // bytes per scale
   static constexpr int S_BYTES = FMT == kQ8 ? 0 : BN * SPR * SB;
-  static constexpr int S_AREA = FMT == kQ8 ? 0 : (S_BYTES < 1024 ? 1024 : S_BYTES);
+  static constexpr int S_AREA = FMT == kQ8 ? 0 : (S_BYTES < 256 * WAVES ? 256 * WAVES : S_BYTES);
   static constexpr int STAGE = A_BYTES + B_BYTES + S_AREA;
-  static constexpr int A_INST = A_BYTES / 1024 / 4;  // direct loads per wave and step
-  static constexpr int B_INST = B_BYTES / 1024 / 4;
-  // dword loads of the step's scales per wave (256 bytes each; with 512
-  // bytes of scales waves 2 and 3 load past the resource into spare LDS)
-  static constexpr int S_INST = FMT == kQ8 ? 0 : (S_BYTES <= 1024 ? 1 : S_BYTES / 1024);
+  static constexpr int A_INST = A_BYTES / 1024 / WAVES;  // direct loads per wave and step
+  static constexpr int B_INST = B_BYTES / 1024 / WAVES;
+  static_assert(A_INST >= 1 && B_INST >= 1, "whole loads per wave");
+  // dword loads of the step's scales per wave (256 bytes each; waves past the
+  // scales load past the resource into spare LDS)
+  static constexpr int S_INST = FMT == kQ8 ? 0 : S_AREA / (256 * WAVES);
   static constexpr int S_RPI = FMT == kQ8 ? 1 : 256 / (SPR * SB);  // rows per scale load
   static constexpr int NL = A_INST + B_INST + S_INST;
 
-  // Tile row (0..127 of the code tile) of B block tn of wave column wn.
+  // Tile row of B block tn of wave column wn.
   static __device__ __forceinline__ int brow(int wn, int tn) {
     if constexpr (PAIR)
-      return (tn >= TN / 2 ? 64 : 0) + wn * (WR / 2) + 16 * (tn % (TN / 2));
+      return (tn >= TN / 2 ? HB : 0) + wn * (WR / 2) + 16 * (tn % (TN / 2));
     return wn * WR + 16 * tn;
   }
 
@@ -138,9 +146,9 @@ struct QGemmDL {
     Src s;
     const int rb = FMT == kQ8 ? p.k : p.k / 2;  // code bytes per weight row
     const int rows = mt.n > n0 ? min(mt.n - n0, NOUT) : 0;
-    // B rows of this wave's code loads: Q8 blocks 2w, 2w + 1 (rows 32 w ..), Q4
-    // rows 32 w ..: the up weight for w >= 2 of a pair
-    const bool up = PAIR && wave >= 2;
+    // the wave's code loads cover rows (BN / WAVES) w ..: the up weight for the
+    // upper half of a pair's waves
+    const bool up = PAIR && wave >= WAVES / 2;
     const char* wb = (const char*)(up ? mt.w2 : mt.w) + (long long)b * mt.w_bstride * 4 +
                      (long long)n0 * rb;
     s.wr = __builtin_amdgcn_make_buffer_rsrc((void*)wb, (short)0, rows * rb, kBufferRsrcWord3);
@@ -161,19 +169,23 @@ struct QGemmDL {
 #pragma unroll
       for (int t = 0; t < B_INST; ++t) {
         const int r = 16 * (wave * B_INST + t) + (lane & 15);
-        s.ob[t] = (PAIR ? (r & 63) : r) * rb + 16 * (lane >> 4);
+        s.ob[t] = (PAIR ? (r & (HB - 1)) : r) * rb + 16 * (lane >> 4);
       }
     } else {
-      const int r = 32 * wave + 16 * (lane >> 5) + (lane & 15);
-      s.ob[0] = (PAIR ? (r & 63) : r) * rb + 16 * ((lane >> 4) & 1);
+#pragma unroll
+      for (int t = 0; t < B_INST; ++t) {
+        const int r = 32 * (wave * B_INST + t) + 16 * (lane >> 5) + (lane & 15);
+        s.ob[t] = (PAIR ? (r & (HB - 1)) : r) * rb + 16 * ((lane >> 4) & 1);
+      }
     }
     if constexpr (FMT == kQ8) {
-      // row scales: wave 0 rows 0-63 (the gate rows of a pair), wave 1 rows
-      // 64-127 (the up rows); fp16: lane i fetches rows 2i, 2i + 1 (lanes 32..
-      // fall past the rows), fp32: row i
+      // row scales: wave w < BN / 64 rows 64 w .. (the up rows of a pair from
+      // HB); fp16: lane i fetches rows 2i, 2i + 1 (lanes 32.. fall past the
+      // rows), fp32: row i
       constexpr int sb = SF16 ? 2 : 4;
-      const bool sup = PAIR && wave == 1;
-      const int base_row = PAIR ? 0 : 64 * (wave & 1);
+      const int w = wave % (BN / 64);
+      const bool sup = PAIR && 64 * w >= HB;
+      const int base_row = PAIR ? (64 * w) % HB : 64 * w;
       const char* sp = (const char*)(sup ? mt.s2 : mt.s) + (long long)b * mt.s_bstride * sb +
                        (long long)(n0 + base_row) * sb;
       const int srows = __builtin_amdgcn_readfirstlane(min(max(rows - base_row, 0), 64));
@@ -188,7 +200,7 @@ struct QGemmDL {
       // row's SPR scales of the step); one weight per wave (the up weight of
       // a pair from row 64)
       const int row0 = S_RPI * wave * S_INST;
-      const bool sup = PAIR && row0 >= 64;
+      const bool sup = PAIR && row0 >= HB;
       const char* sp = (const char*)(sup ? mt.s2 : mt.s) +
                        ((long long)b * mt.s_bstride + (long long)n0 * p.groups_per_row) * SB;
       s.sr = __builtin_amdgcn_make_buffer_rsrc((void*)sp, (short)0,
@@ -198,26 +210,29 @@ struct QGemmDL {
         const int j = wave * S_INST + i;  // load index over the workgroup
         const int byte = 256 * j + 4 * lane;  // in the step's scale block [row][SPR]
         const int srow = byte / (SPR * SB), sin = byte % (SPR * SB);
-        const int wrow = PAIR ? (srow & 63) : srow;
+        const int wrow = PAIR ? (srow & (HB - 1)) : srow;
         s.os[i] = 256 * j >= S_BYTES ? (1 << 30) : wrow * p.groups_per_row * SB + sin;
       }
     }
     return s;
   }
 
-  // The direct loads of step st into the LDS stage at byte `base`.
-  static __device__ __forceinline__ void issue(const Src& s, uint32_t base, int wave, int st) {
+  // The direct loads of step st into the LDS stage at byte `base`; !live: the
+  // same loads past the resources (zeros, no traffic).
+  static __device__ __forceinline__ void issue(const Src& s, uint32_t base, int wave, int st,
+                                               bool live = true) {
+    const int dead = live ? 0 : 1 << 30;
 #pragma unroll
     for (int t = 0; t < A_INST; ++t)
-      dma<16>(s.xr, base + (wave * A_INST + t) * 1024, s.oa[t] + st * RA);
+      dma<16>(s.xr, base + (wave * A_INST + t) * 1024, s.oa[t] + (st * RA + dead));
 #pragma unroll
     for (int t = 0; t < B_INST; ++t)
-      dma<16>(s.wr, base + A_BYTES + (wave * B_INST + t) * 1024, s.ob[t] + st * CP);
+      dma<16>(s.wr, base + A_BYTES + (wave * B_INST + t) * 1024, s.ob[t] + (st * CP + dead));
     if constexpr (FMT == kQ4) {
 #pragma unroll
       for (int i = 0; i < S_INST; ++i)
         dma<4>(s.sr, base + A_BYTES + B_BYTES + (wave * S_INST + i) * 256,
-               s.os[i] + st * SPR * SB);
+               s.os[i] + (st * SPR * SB + dead));
     }
   }
 
@@ -243,13 +258,13 @@ struct QGemmDL {
     int s_off;     // scale offset (row l16, the lane group's scale group) inside block row 0
   };
 
-  static __device__ __forceinline__ Lane lane_offsets(int lane) {
+  static __device__ __forceinline__ Lane lane_offsets(int lane, int wm) {
     Lane L;
     const int l16 = lane & 15, lk = lane >> 4;
     const int f = aswz(l16);
 #pragma unroll
     for (int kk = 0; kk < NE; ++kk)
-      L.a_off[kk] = l16 * RA + (((PERM ? NE * lk + kk : 4 * kk + lk) ^ f) << 4);
+      L.a_off[kk] = (wm * 16 * TM + l16) * RA + (((PERM ? NE * lk + kk : 4 * kk + lk) ^ f) << 4);
     // 16-byte code reads (C16): [quarter][row] per 16-row block, lane l at 16 l.
     // Q4 codes [half][row] per 16-row block: FD chunks 2 lk, 2 lk + 1 (half
     // lk / 2, bytes 8 (lk % 2) ..); exact: dword lk of each half (+ 256 kk)
@@ -266,6 +281,36 @@ struct QGemmDL {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
       a[tm] = *(const f16x8*)(base + 16 * tm * RA + L.a_off[kk]);
+  }
+
+  // VALU instructions of a B fragment's expansion
+  static constexpr int EXPAND_VALU = FMT == kQ8 ? 8 : 17;
+  // The B fragments of K extent kk (Q8, or Q4 as fp16 weight tiles).
+  static __device__ __forceinline__ void expand_b(int kk, const Frag& f, f16x8 (&b)[TN]) {
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      uint32_t e[4];
+      if constexpr (FMT == kQ8) {
+        q8_pairs(f.c[tn][2 * kk], e[0], e[1]);
+        q8_pairs(f.c[tn][2 * kk + 1], e[2], e[3]);
+      } else {
+        q4_pairs_seq(f.c[tn][kk], e);
+        const f16 s16 = (f16)scale_of(f.s[tn][kk * NS / NE], SF16);
+        const f16x2 s2 = {s16, s16};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = as_u(as_h2(e[j]) * s2);
+      }
+      b[tn] = pack8(e[0], e[1], e[2], e[3]);
+    }
+  }
+  // The MFMAs of activation fragments a with B fragments b.
+  static __device__ __forceinline__ void mfma_ab(const f16x8 (&a)[TM], const f16x8 (&b)[TN],
+                                                 f32x4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+        acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[tm], b[tn], acc[tm][tn], 0, 0, 0);
   }
 
   static __device__ __forceinline__ void read_b(const char* base, const Lane& L, int wn, Frag& f) {
@@ -369,29 +414,34 @@ struct QGemmDL {
   // cache) small, and the stores cover whole rows of the tile.
   static constexpr int CW = BN + 4;            // floats per LDS row of C
   static constexpr int TPR = NOUT / 8;         // threads per output row
-  static constexpr int RPP = kThreads / TPR;   // rows per pass
+  static constexpr int RPP = THREADS / TPR;    // rows per pass
   static constexpr int C_BYTES = 64 * CW * 4;
 
   // Rows 64 h .. 64 h + 63 of the tile's raw accumulators into C, then a
   // barrier (a barrier first for h > 0: every thread has read the last half).
-  static __device__ __forceinline__ void stage_c(int h, int lane, int wn,
+  static __device__ __forceinline__ void stage_c(int h, int lane, int wm, int wn,
                                                  const f32x4 (&acc)[TM][TN], float* C) {
     const int l16 = lane & 15, lk = lane >> 4;
     if (h > 0) bar();
+    constexpr int HW = TM / 4;  // 64-row pieces per wave
 #pragma unroll
-    for (int tq = 0; tq < 4; ++tq)
+    for (int hw = 0; hw < HW; ++hw)
+      if (h == wm * HW + hw) {
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
+        for (int tq = 0; tq < 4; ++tq)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          C[(16 * tq + 4 * lk + r) * CW + brow(wn, tn) + l16] = acc[4 * h + tq][tn][r];
+          for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              C[(16 * tq + 4 * lk + r) * CW + brow(wn, tn) + l16] = acc[4 * hw + tq][tn][r];
+      }
     wait_lgkm0();
     bar();
   }
 
   static __device__ __forceinline__ void finish(const QmvParams& p, const QmvMat& mt, int b,
-                                                int n0, int m0, int tid, int lane, int wn, const f32x4 (&acc)[TM][TN], float* C,
-                                                const char* qs) {
+                                                int n0, int m0, int tid, int lane, int wm, int wn,
+                                                const f32x4 (&acc)[TM][TN], float* C, const char* qs) {
     const int l16 = lane & 15, lk = lane >> 4;
     // everything the loops below use, in registers (see sreg)
     const EpiArgs E = epi_args(p);
@@ -425,20 +475,20 @@ struct QGemmDL {
       rs1[j] = 1.0f;
       if constexpr (FMT == kQ8) {
         // row scales as the prologue placed them: tile row r at (r / 64) * 512
-        // + (r % 64) * (2 or 4) bytes; the up half of a pair from row 64
+        // + (r % 64) * (2 or 4) bytes; the up half of a pair from row HB
         const int r = 8 * cg + j;
         rs0[j] = scale_of(SF16 ? *(const uint16_t*)(qs + (r >> 6) * 512 + (r & 63) * 2)
                                : *(const uint32_t*)(qs + (r >> 6) * 512 + (r & 63) * 4),
                           SF16);
         if constexpr (PAIR)
-          rs1[j] = scale_of(SF16 ? *(const uint16_t*)(qs + 512 + r * 2)
-                                 : *(const uint32_t*)(qs + 512 + r * 4),
+          rs1[j] = scale_of(SF16 ? *(const uint16_t*)(qs + (HB / 64 + (r >> 6)) * 512 + (r & 63) * 2)
+                                 : *(const uint32_t*)(qs + (HB / 64 + (r >> 6)) * 512 + (r & 63) * 4),
                             SF16);
       }
     }
 #pragma unroll
     for (int h = 0; h < BM / 64; ++h) {
-      stage_c(h, lane, wn, acc, C);
+      stage_c(h, lane, wm, wn, acc, C);
 #pragma unroll 1
       for (int row = r0; row < 64; row += RPP) {
         const int m = m0 + 64 * h + row;
@@ -447,8 +497,8 @@ struct QGemmDL {
         *(f32x4*)&g[0] = *(const f32x4*)&C[row * CW + 8 * cg];
         *(f32x4*)&g[4] = *(const f32x4*)&C[row * CW + 8 * cg + 4];
         if constexpr (PAIR) {
-          *(f32x4*)&u[0] = *(const f32x4*)&C[row * CW + 64 + 8 * cg];
-          *(f32x4*)&u[4] = *(const f32x4*)&C[row * CW + 64 + 8 * cg + 4];
+          *(f32x4*)&u[0] = *(const f32x4*)&C[row * CW + HB + 8 * cg];
+          *(f32x4*)&u[4] = *(const f32x4*)&C[row * CW + HB + 8 * cg + 4];
         }
         float res[8];
 #pragma unroll
@@ -531,7 +581,7 @@ struct QGemmDL {
   // into partial plane c, through C as in finish: 8 consecutive partials of
   // a row per thread, two 16-byte stores where the plane is aligned.
   static __device__ __forceinline__ void spill(const QmvParams& p, const QmvMat& mt, int b,
-                                               int n0, int m0, int tid, int lane, int wn, int c,
+                                               int n0, int m0, int tid, int lane, int wm, int wn, int c,
                                                const f32x4 (&acc)[TM][TN], float* C) {
     constexpr int NW = PAIR ? 2 : 1;
     const int nst = sreg(mt.n_store), mn = sreg(mt.n), pm = sreg(p.m);
@@ -543,15 +593,15 @@ struct QGemmDL {
     const bool vec = nb + 8 <= mn && (nst & 3) == 0 && ((uintptr_t)base & 15) == 0;
 #pragma unroll
     for (int h = 0; h < BM / 64; ++h) {
-      stage_c(h, lane, wn, acc, C);
+      stage_c(h, lane, wm, wn, acc, C);
 #pragma unroll 1
       for (int row = r0; row < 64; row += RPP) {
         const int m = m0 + 64 * h + row;
         if (m >= pm) continue;
 #pragma unroll
         for (int hh = 0; hh < NW; ++hh) {
-          const f32x4 v0 = *(const f32x4*)&C[row * CW + 64 * hh + 8 * cg];
-          const f32x4 v1 = *(const f32x4*)&C[row * CW + 64 * hh + 8 * cg + 4];
+          const f32x4 v0 = *(const f32x4*)&C[row * CW + HB * hh + 8 * cg];
+          const f32x4 v1 = *(const f32x4*)&C[row * CW + HB * hh + 8 * cg + 4];
           const long long o = ((long long)m * NW + hh) * nst + nb;
           if (vec) {
             *(gf32x4*)(gb + o * 4) = v0;
@@ -608,14 +658,74 @@ __device__ __forceinline__ void qgemm_dl_step(const typename G::Src& src, const 
   f = g;
 }
 
-template <int FMT, int BM, bool PAIR, bool SF16, int G, bool FD, int WPE, int KS = 64, int NST = 3>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WPE)))
+// A scheduling group of n MFMAs (mask 0x8), VALU (0x2) or LDS reads (0x100).
+#define AEXQ_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
+
+// The step of the eight-wave tiles (Q8, Q4 as fp16 weight tiles).  Each extent's
+// MFMAs run with fragments that are already there -- a[] and b[] on entry -- and
+// between them the wave reads the next extent's activations and expands its
+// codes: with one workgroup per CU the waves meet at every barrier, and reads,
+// expansion and MFMAs would add up.  Every step issues its loads, past
+// the end as well (no traffic), so that one constant wait serves them all and the
+// step is one block of code.
+template <typename G, int NST>
+__device__ __forceinline__ void qgemm_dl_step8(const typename G::Src& src, const typename G::Lane& L,
+                                               char* cur, char* nxt, int wave, int wn, int st, int s1,
+                                               typename G::Frag& f, f16x8 (&b)[G::TN],
+                                               f32x4 (&acc)[G::TM][G::TN]) {
+  constexpr int NM = G::TM * G::TN;                         // MFMAs of an extent
+  constexpr int NV = (G::EXPAND_VALU * G::TN + NM - 1) / NM;  // VALU to place after each
+#pragma unroll
+  for (int kk = 0; kk < G::NE; ++kk) {
+    f16x8 a1[G::TM], b1[G::TN];
+    const bool last = kk == G::NE - 1;
+    if (!last) {
+      G::read_a(cur, L, kk + 1, a1);
+      G::expand_b(kk + 1, f, b1);
+      G::mfma_ab(f.a, b, acc);
+      AEXQ_SGB(0x100, G::TM);
+#pragma unroll
+      for (int i = 0; i < NM; ++i) {
+        AEXQ_SGB(0x8, 1);
+        AEXQ_SGB(0x2, NV);
+      }
+    } else {
+      // this step's fragments are in registers before any wave refills `cur`;
+      // step st + 1's loads have landed
+      wait_lgkm0();
+      wait_vm<(NST - 2) * G::NL>();
+      bar();
+      G::issue(src, lds_addr(cur), wave, st + NST, st + NST < s1);
+      G::read_b(nxt, L, wn, f);
+      G::read_a(nxt, L, 0, a1);
+      G::mfma_ab(f.a, b, acc);
+      G::expand_b(0, f, b1);
+      AEXQ_SGB(0x100, G::TM + 3 * G::TN);
+      constexpr int lead = NM * 3 / 8;
+      AEXQ_SGB(0x8, lead);
+#pragma unroll
+      for (int i = lead; i < NM; ++i) {
+        AEXQ_SGB(0x8, 1);
+        AEXQ_SGB(0x2, (G::EXPAND_VALU * G::TN + NM - lead - 1) / (NM - lead));
+      }
+    }
+#pragma unroll
+    for (int tm = 0; tm < G::TM; ++tm) f.a[tm] = a1[tm];
+#pragma unroll
+    for (int tn = 0; tn < G::TN; ++tn) b[tn] = b1[tn];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+template <int FMT, int BM, bool PAIR, bool SF16, int G, bool FD, int WPE, int KS = 64, int NST = 3,
+          int WM = 1>
+__global__ __launch_bounds__(256 * WM) __attribute__((amdgpu_waves_per_eu(WPE)))
 void qgemm_dl_kernel(const QmvParams p, int mtiles) {
-  using Q = QGemmDL<FMT, BM, PAIR, SF16, G, FD, KS>;
+  using Q = QGemmDL<FMT, BM, PAIR, SF16, G, FD, KS, WM>;
   static_assert(NST == 2 || NST == 3, "a ring of two or three LDS stages");
   static_assert(Q::C_BYTES <= NST * Q::STAGE, "the accumulator tile reuses the stages");
   __shared__ __align__(1024) char lds[NST * Q::STAGE];
-  __shared__ __align__(16) char qs[FMT == kQ8 ? 1024 : 16];  // Q8 row scales of the tile
+  __shared__ __align__(16) char qs[FMT == kQ8 ? 8 * Q::BN : 16];  // Q8 row scales of the tile
   char* const sg[3] = {lds, lds + Q::STAGE, lds + (NST - 1) * Q::STAGE};
   // weight tile tn, row tile tm and K chunk kc of this workgroup (the chunks
   // of a split K sit next to each other on one XCD); readfirstlane keeps the
@@ -640,13 +750,13 @@ void qgemm_dl_kernel(const QmvParams p, int mtiles) {
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wn = wave;  // the wave's 32 weight rows
+  const int wm = WM == 1 ? 0 : wave >> 2, wn = WM == 1 ? wave : wave & 3;
   const int steps = p.k / Q::BK;
   const int cs = S > 1 ? p.sk_cs : steps;
   const int s0 = kc * cs, s1 = min(s0 + cs, steps);  // this workgroup's K steps
   if (s0 >= s1) return;
   const typename Q::Src src = Q::source(p, mt, b, n0, m0, lane, wave);
-  const typename Q::Lane L = Q::lane_offsets(lane);
+  const typename Q::Lane L = Q::lane_offsets(lane, wm);
 
   f32x4 acc[Q::TM][Q::TN];
 #pragma unroll
@@ -656,19 +766,36 @@ void qgemm_dl_kernel(const QmvParams p, int mtiles) {
 
   // prologue: steps s0 .. s0 + NST - 1 in flight, step s0 landed and its
   // first fragments read
-  // Q8: the tile's row scales go to LDS with the first step (waves 0 and 1:
-  // rows 0-63 and 64-127, or the gate and up rows of a pair)
+  // Q8: the tile's row scales go to LDS with the first step
   if constexpr (FMT == kQ8)
-    if (S == 1 && wave < 2) dma<4>(src.sr, lds_addr(qs) + wave * 512, src.os[0]);
+    if (S == 1 && wave < Q::BN / 64) dma<4>(src.sr, lds_addr(qs) + wave * 512, src.os[0]);
 #pragma unroll
   for (int i = 0; i < NST; ++i)
-    if (s0 + i < s1) Q::issue(src, lds_addr(sg[i]), wave, s0 + i);
+    if (WM > 1 || s0 + i < s1) Q::issue(src, lds_addr(sg[i]), wave, s0 + i, s0 + i < s1);
   // (the row scales, issued first, have landed with step s0)
-  wait_steps<Q::NL, NST - 1>(s1 - s0 - 1);
+  wait_steps<Q::NL, NST - 1>(WM > 1 ? NST - 1 : s1 - s0 - 1);
   bar();
   typename Q::Frag f;
   Q::read_a(sg[0], L, 0, f.a);
   Q::read_b(sg[0], L, wn, f);
+  if constexpr (WM > 1) {
+    static_assert(WM == 1 || FMT == kQ8 || FD, "eight-wave tiles: Q8 or fp16 weight tiles");
+    f16x8 b0[Q::TN];
+    Q::expand_b(0, f, b0);
+    int st = s0;
+    for (int it = (s1 - s0) / NST; it > 0; --it) {
+#pragma unroll
+      for (int i = 0; i < NST; ++i)
+        qgemm_dl_step8<Q, NST>(src, L, sg[i], sg[(i + 1) % NST], wave, wn, st + i, s1, f, b0, acc);
+      st += NST;
+    }
+    const int tail = s1 - st;
+#pragma unroll
+    for (int i = 0; i < NST - 1; ++i)
+      if (tail > i)
+        qgemm_dl_step8<Q, NST>(src, L, sg[i], sg[i + 1], wave, wn, st + i, s1, f, b0, acc);
+    wait_vm<0>();  // the loads past the end, before the stages become C
+  } else {
   // NST steps per iteration: the stages rotate with compile-time names
   int st = s0;
   for (int it = (s1 - s0) / NST; it > 0; --it) {
@@ -681,12 +808,13 @@ void qgemm_dl_kernel(const QmvParams p, int mtiles) {
 #pragma unroll
   for (int i = 0; i < NST - 1; ++i)
     if (tail > i) qgemm_dl_step<Q, NST>(src, L, sg[i], sg[i + 1], wave, wn, st + i, s1, f, acc);
+  }
   wait_lgkm0();  // the last fragments are read before the stages become C
   bar();
   if (S == 1)
-    Q::finish(p, mt, b, n0, m0, threadIdx.x, lane, wn, acc, (float*)lds, qs);
+    Q::finish(p, mt, b, n0, m0, threadIdx.x, lane, wm, wn, acc, (float*)lds, qs);
   else
-    Q::spill(p, mt, b, n0, m0, threadIdx.x, lane, wn, kc, acc, (float*)lds);
+    Q::spill(p, mt, b, n0, m0, threadIdx.x, lane, wm, wn, kc, acc, (float*)lds);
 }
 
 }  // namespace aexq

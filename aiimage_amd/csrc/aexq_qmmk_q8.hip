@@ -49,7 +49,7 @@ static constexpr int kRingLds = 152 * 1024;
 // us): N = 1024, K = 2048, M = 16: 5.4 / 5.2 against 8.8 / 7.9 on the MFMA
 // block kernels with their split-K fix-up, M = 64: 5.9 / 5.7 against 10.4 / 9.9
 // on the tiled GEMM, M = 512: 9.9 / 9.5 against 23.8 / 23.2.
-bool qmmk_pick(int m, long long t16, bool pair, bool rag, int* mt, int* nt, int* waves) {
+bool qmmk_pick(int m, long long t16, bool q8, bool pair, bool rag, int* mt, int* nt, int* waves) {
   const long long m16 = (m + 15) / 16, m32 = (m + 31) / 32, m64 = (m + 63) / 64;
   const long long t32 = (t16 + 1) / 2;
   auto take = [&](int a, int b, int w) {
@@ -78,6 +78,10 @@ bool qmmk_pick(int m, long long t16, bool pair, bool rag, int* mt, int* nt, int*
     }
     return t32 <= 512 && take(2, 2, 8);
   }
+  // Q8 from 96 tiles of 128 x 128: the tiled GEMM's eight-wave form (512 x 3072 x
+  // 1024: 18.8 us against 21.1; Q4, which expands its codes twice there, 22.0
+  // against 21.6)
+  if (q8 && m > 64 && (t16 + (pair ? 3 : 7)) / (pair ? 4 : 8) * ((m + 127) / 128) >= 96) return false;
   if (!pair && t16 * m16 <= 640) return take(2, 1, 8);  // 1024 x 2048, M = 128: 6.7 us; 2:2 7.2
   if (t32 * m32 <= 256) return take(2, 2, 8);           // 4096 x 4096, M = 64: 9.9 us; 4 waves 10.9
   // more workgroups than CUs: four waves each, several workgroups per CU

@@ -78,7 +78,7 @@ CASES = [
     ("q8h", 33, 1001, 1024, "plain", "qgemmk"), ("q4h", 64, 1024, 3584, "plain", "qgemmk"),
     ("q4g16h", 65, 515, 512, "plain", "qgemmk"), ("q4s", 97, 3000, 640, "plain", "qgemmk"),
     ("q8s", 130, 4100, 1024, "plain", "qgemmk"), ("q4g16s", 257, 4096, 1024, "plain", "qgemmk"),
-    ("q4h", 500, 1024, 2048, "residual", "qgemmk"), ("q8h", 385, 3072, 1024, "residual", "qgemmk"),
+    ("q4h", 500, 1024, 2048, "residual", "qgemmk"), ("q8h", 300, 3072, 1024, "residual", "qgemmk"),
     # SwiGLU pairs; RMSNorm-in: one slice a wave, whole rows in the ring, past it
     ("q4h", 5, 3584, 1024, "swiglu", "qmmk"), ("q8h", 31, 3000, 2048, "swiglu", "qmmk"),
     ("q4g16h", 32, 5200, 1024, "swiglu", "qmmk"), ("q8s", 16, 130, 4096, "rms", "qmmk"),
