@@ -10,6 +10,7 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -63,13 +64,18 @@ def build(verbose: bool = True, jobs: int = 4, stamps: bool = False) -> str:
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         objs.append(obj)
         cmd = [cc, *flags(), *extra, "-c", path, "-o", obj]
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
-        while len([p for _, p in procs if p.poll() is None]) >= jobs:
+        # (a file, not a pipe: a compiler whose output fills a pipe that is read
+        # only at the end would wait for ever, and hold up the ones behind it)
+        out = tempfile.TemporaryFile()
+        procs.append((src, subprocess.Popen(cmd, stdout=out, stderr=subprocess.STDOUT), out))
+        while len([p for _, p, _ in procs if p.poll() is None]) >= jobs:
             time.sleep(0.2)
     failed = []
-    for src, p in procs:
-        out, _ = p.communicate()
-        text = out.decode(errors="replace")
+    for src, p, out in procs:
+        p.wait()
+        out.seek(0)
+        text = out.read().decode(errors="replace")
+        out.close()
         if p.returncode != 0:
             failed.append((src, text))
         elif verbose and "error" in text.lower():
