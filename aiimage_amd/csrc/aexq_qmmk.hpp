@@ -29,7 +29,8 @@
 //    v_permlane16_swap per 16 bytes): MFMA e then covers codes 32 e .. 32 e +
 //    31, and its product is scaled in fp32 into the accumulator, so the weight
 //    is exactly float(q) * scale.  Groups of 16: two MFMAs per extent, each
-//    with the other group's lanes zeroed.
+//    with the other group's activations zeroed (not its codes: an infinite
+//    activation times a zeroed code would be NaN in every output).
 // The activation fragments are read in the same order.
 //
 // RMSNorm-in (RMS): the workgroup holds whole activation rows, so it forms
@@ -313,11 +314,11 @@ struct QmmK {
           const float s0 = sc[2 * e], s1 = sc[2 * e + 1];
           const bool first = lane < 32;
           const f16x8 zero = {};
-          const f16x8 b0 = first ? bq : zero, b1 = first ? zero : bq;
 #pragma unroll
           for (int m = 0; m < MT; ++m) {
-            const f32x4 v0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[m][e], b0, z, 0, 0, 0);
-            const f32x4 v1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[m][e], b1, z, 0, 0, 0);
+            const f16x8 x0 = first ? x[m][e] : zero, x1 = first ? zero : x[m][e];
+            const f32x4 v0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x0, bq, z, 0, 0, 0);
+            const f32x4 v1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(x1, bq, z, 0, 0, 0);
             acc[m][t] = __builtin_elementwise_fma(f32x4{s0, s0, s0, s0}, v0, acc[m][t]);
             acc[m][t] = __builtin_elementwise_fma(f32x4{s1, s1, s1, s1}, v1, acc[m][t]);
           }

@@ -191,6 +191,34 @@ def test_ragged_k_keeps_to_its_row(ctx, aexq, orc, fmt):
     assert normwise(got[:, rest], ref) <= TOL32
 
 
+@pytest.mark.parametrize("fmt,m,k", [("q4g16h", 5, 1024), ("q4g16s", 20, 1024),
+                                     ("q4g16h", 20, 1040), ("q4h", 5, 1024), ("q8h", 5, 1024)])
+def test_infinite_activation_keeps_its_sign(ctx, aexq, orc, fmt, m, k):
+    """An infinite activation gives +-inf by the sign of its code (NaN where the
+    code is 0) in its own row, in exact products as in float64, and leaves the
+    other rows alone."""
+    print(f"[gpu-case] wave split infinite x {fmt} m={m} k={k}", flush=True)
+    from aiimage_amd import synth
+    n, row = 200, 3
+    w, wf = _weight(ctx, aexq, orc, fmt, n, k, 12)
+    x16 = synth.activations(m, k, 4)
+    x16[row, k - 9] = np.inf
+    y = aexq.new_activation(m, n, torch.float32, aexq.LAYOUT_LINEAR)
+    xd, yd = aexq.describe(dev(x16), m, k), aexq.describe(y, m, n)
+    plan = ctx.plan_check(w, xd, yd)
+    assert plan.startswith("kernel=qmmk "), plan
+    ctx.linear(w, xd, yd)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(m, n)
+    wx = np.asarray(for_plan(wf, plan), np.float64)[:, k - 9]
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_array_equal(got[row], np.inf * wx)
+    rest = [r for r in range(m) if r != row]
+    ref = orc.gemm_gpu_semantics(np.ascontiguousarray(x16[rest]).astype(np.float32),
+                                 for_plan(wf, plan))
+    assert normwise(got[rest], ref) <= TOL32
+
+
 def test_other_kernels_where_they_stay(ctx, aexq, orc):
     """Forms the wave-split kernel does not take: one row and short ragged rows
     stream, K of odd 64s is tiled, fp32 rows and other groups go where they went."""
