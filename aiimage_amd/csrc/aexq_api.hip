@@ -1136,6 +1136,8 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
     if (M > 32)
       for (const char* name : {"AEXQ_QGEMM_OFF", "AEXQ_QGEMM_BM", "AEXQ_QGEMM_K64"})
         if (getenv(name)) return;
+    // (a tile's up to 64 activation and residual rows are at 32-bit byte offsets)
+    if (xv.rstride >= 1 << 23 || ((a.flags & AEXQ_EPI_RESIDUAL_ADD) && rv.rstride >= 1 << 22)) return;
     const bool fused = rms_in && (rag || M <= 32) && getenv("AEXQ_RMS_PREPASS") == nullptr;
     // (the kernel reads gamma[0 .. K) of fp16 rows)
     if (fused ? !(rms_ok && x_ok) : !x_ok && !rms_in) return;

@@ -219,6 +219,29 @@ def test_infinite_activation_keeps_its_sign(ctx, aexq, orc, fmt, m, k):
     assert normwise(got[rest], ref) <= TOL32
 
 
+def test_rows_too_far_apart_for_its_offsets(ctx, aexq, orc):
+    """Row strides whose tile passes 32-bit offsets keep the kernels they had."""
+    print("[gpu-case] wave split row strides", flush=True)
+    m, n, k = 2, 64, 1024
+    w, _ = _weight(ctx, aexq, orc, "q8h", n, k, 2)
+    x = torch.zeros(m * k, dtype=torch.float16, device="cuda")
+    y = aexq.new_activation(m, n, torch.float16, aexq.LAYOUT_LINEAR)
+
+    def rows_of(t, width, stride):   # tiled storage of one tile row, wider than the matrix
+        d = aexq.describe(t, m, width)
+        d.layout, d.storage = aexq.LAYOUT_PACK4_TILED, type(d.storage)(3, stride // 4, m, 1, 4)
+        return d
+
+    def kernel(xs, rs):   # (planned only: rows that far apart are not there)
+        yd = rows_of(y, n, rs)
+        return ctx.plan_check(w, rows_of(x, k, xs), yd, residual=yd).split()[0]
+
+    assert kernel(k, n) == "kernel=qmmk"
+    assert kernel((1 << 23) - 8, (1 << 22) - 8) == "kernel=qmmk"
+    assert kernel(1 << 23, n) != "kernel=qmmk"
+    assert kernel(k, 1 << 22) != "kernel=qmmk"
+
+
 def test_other_kernels_where_they_stay(ctx, aexq, orc):
     """Forms the wave-split kernel does not take: one row and short ragged rows
     stream, K of odd 64s is tiled, fp32 rows and other groups go where they went."""
