@@ -88,8 +88,8 @@ hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, v
 // ---------------------------------------------------------------------------
 // GQA decode attention in one launch.  Workgroup (kv head g, split c) covers
 // `per` positions (a multiple of 64) of the `len` cached ones for the G = hq /
-// hkv query heads of g, so every cached K and V row is read once.  Its four
-// waves run by themselves, 16 positions of each 64 per wave, with a running
+// hkv query heads of g, so every cached K and V row is read once.  Its waves
+// (four or eight) run by themselves, 16 positions of each 64 per wave, with a running
 // maximum each and no barrier until the end:
 //   scores   lanes 4i..4i+3 own position i of the wave's 16, lane 4i + j the
 //            dims 32 r + 8 j + [0, 8) for r < 4 (so one load instruction covers
@@ -101,7 +101,8 @@ hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, v
 //            its own DPP row (row_newbcast), lane l the dims 8 (l % 16) + [0, 8):
 //            four 16-byte loads cover the wave's 16 rows.
 // The next pass's K and V rows are requested before the current ones'
-// products (eight waves for splits of more than one four-wave pass), and q (rotated here when RoPE is fused) meets K after one barrier.
+// products (eight waves for splits of more than one four-wave pass), and q
+// (rotated here when RoPE is fused) meets K after one barrier.
 // The waves' (max, sum, acc) meet in LDS; the split's go to part[h][split].
 // The last workgroup of kv head g to finish (a device-scope counter that the
 // same workgroup resets to 0, so the launch needs no clearing and replays
@@ -109,8 +110,8 @@ hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, v
 //   M = max m_s, L = sum l_s e^(m_s - M), out = sum acc_s e^(m_s - M) / max(L, 1e-20).
 // That merge reads splits x G rows of 528 bytes through one CU, so a long cache
 // takes longer splits rather than more of them (attn_splits): with 64 positions
-// a split, 16 heads over 4 x 16384 positions took 22.6 us, half of them in the
-// merge, now 14.6 (32 MB: 5 us at the rate the shared cache level gives); up to
+// a split, 16 heads over 4 x 16384 positions took 21.0 us, half of them in the
+// merge, now 13.1 (32 MB: 5 us at the rate the shared cache level gives); up to
 // 64 positions there is one split and nothing to merge (7.4 -> 5.0 us).
 // head_dim == 128.
 // ---------------------------------------------------------------------------
