@@ -134,27 +134,39 @@ constexpr int kAttnCounterStride = 64;
 constexpr int kAttnMaxSplits = 64;   // combine staging in LDS
 constexpr int kAttnMaxLen = 32768;   // positions a launch takes
 
+// LDS of a workgroup of W waves.
 template <int G, int W>
-__global__ __launch_bounds__(64 * W) void attn_decode_kernel(
-    const f16* q, const f16* kcache, const f16* vcache, int cap, int len, float scale,
-    int splits, float* part, int* counters, f16* out, const f16* knew, const f16* vnew,
-    f16* kcache_w, f16* vcache_w, const float* cosv, const float* sinv, const int* posp) {
+struct AttnLds {
+  // P V sums: the waves of a split, then the merge's row groups
+  alignas(16) float pv[2 * W][G][kAttnDim];
+  alignas(16) f16 qs[G][kAttnDim];
+  alignas(16) f16 kn[kAttnDim];
+  alignas(16) f16 vn[kAttnDim];
+  float wm[W][G], wl[W][G];
+  float cm[G * kAttnMaxSplits];  // split maxima, then weights
+  float cl[G * kAttnMaxSplits];  // split sums
+  float hl[G];
+  int last;
+};
+
+// Passes of a split, where the launch knows them: one, several, or either (a
+// device-side position).  Code for one pass alone starts sooner: 16/4 heads at
+// 1024 positions 6.5 us with both forms in the kernel, 6.3 with one.
+enum AttnPasses { kOnePass, kManyPasses, kAnyPasses };
+
+template <int G, int W, AttnPasses PASSES>
+__device__ __forceinline__ void attn_decode(
+    AttnLds<G, W>& lds, const f16* q, const f16* kcache, const f16* vcache, int cap, int len,
+    float scale, int splits, float* part, int* counters, f16* out, const f16* knew, const f16* vnew,
+    f16* kcache_w, f16* vcache_w, const float* cosv, const float* sinv) {
   const int g = blockIdx.x, c = blockIdx.y;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   constexpr int half = kAttnDim / 2;
   constexpr int T = 64 * W;     // threads
   constexpr int P = 16 * W;     // positions of one pass
   constexpr int RG = T / 32;    // row groups of the merge
-  if (posp) {
-    // decode position in device memory (a captured graph advances it): the
-    // grid covers the cache capacity, the tables hold [cap][half] rows
-    const int pp = min(max(*posp, 0), cap - 1);
-    len = pp + 1;
-    cosv += (long long)pp * half;
-    sinv += (long long)pp * half;
-  }
   // positions per split: the live length over the grid's splits
-  const int per = ((len + splits - 1) / splits + P - 1) / P * P;
+  const int per = PASSES == kOnePass ? P : ((len + splits - 1) / splits + P - 1) / P * P;
   const int live_splits = (len + per - 1) / per;
   const int p0 = c * per, p1 = min(p0 + per, len);
   const int pl = t >> 2, qq = t & 3;  // scores: position p0 + pl of a pass, dims 32 r + 8 qq ..
@@ -162,10 +174,10 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
   const int pos = len - 1;             // the appended position when RoPE is fused
   const bool has_new = rope && pos >= p0 && pos < p0 + per;
   const long long head_off = (long long)g * cap * kAttnDim;
-  // P V sums: the waves of a split, then the merge's row groups
-  __shared__ __align__(16) float pv[RG][G][kAttnDim];
-  __shared__ float wm[W][G], wl[W][G];
-  __shared__ int last;
+  auto& pv = lds.pv;
+  auto& wm = lds.wm;
+  auto& wl = lds.wl;
+  int& last = lds.last;
   if (c >= live_splits) {
     // a split past the live length (the grid was sized for the capacity):
     // nothing to score, but it still counts in so the merge starts once
@@ -234,9 +246,9 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
 
     // 2. q of the G heads (rotated and rounded to fp16 when RoPE is fused) and,
     // in the split that holds it, the appended K/V row
-    __shared__ __align__(16) f16 qs[G][kAttnDim];
-    __shared__ __align__(16) f16 kn[kAttnDim];
-    __shared__ __align__(16) f16 vn[kAttnDim];
+    auto& qs = lds.qs;
+    auto& kn = lds.kn;
+    auto& vn = lds.vn;
 #pragma unroll
     for (int r = 0; r < QI; ++r) {
       const int i = t + r * T;
@@ -349,7 +361,7 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
       }
     };
     // a split of one pass, with no rows of a next one on the way
-    if (per == P) {
+    if (PASSES == kOnePass || (PASSES == kAnyPasses && per == P)) {
       take(p0, cur, std::true_type{});
     } else {
       for (int q0 = p0; q0 < p1; q0 += P) {
@@ -432,8 +444,9 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
   // pitch (`splits`); only the first live_splits of each head hold partials
   // of this launch.
   const int nsp = live_splits;
-  __shared__ float cm[G * kAttnMaxSplits];  // split maxima, then weights
-  __shared__ float cl[G * kAttnMaxSplits];  // split sums
+  auto& cm = lds.cm;
+  auto& cl = lds.cl;
+  auto& hl = lds.hl;
   const int rows = G * splits;
   const float* pg = part + (long long)g * rows * kAttnStride;
   const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
@@ -468,8 +481,7 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
                : 0.0f;
   }
   __syncthreads();
-  // per head: M = max m_s (each wave reduces the heads h == wave mod 4)
-  __shared__ float hm[G], hl[G];
+  // per head: M = max m_s (each wave reduces the heads h == wave mod W)
   for (int h = wave; h < G; h += W) {
     float m = -INFINITY;
     for (int s2 = lane; s2 < nsp; s2 += 64) m = fmaxf(m, cm[h * splits + s2]);
@@ -481,10 +493,7 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
       l = fmaf(cl[h * splits + s2], w, l);
     }
     l = wave_sum(l);
-    if (lane == 0) {
-      hm[h] = m;
-      hl[h] = l;
-    }
+    if (lane == 0) hl[h] = l;
   }
   __syncthreads();
   float ac[G][4];
@@ -521,6 +530,39 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
     out[((long long)g * G + h) * kAttnDim + dd] = (f16)(a / fmaxf(hl[h], 1e-20f));
   }
   if (t == 0) counters[g * kAttnCounterStride] = 0;  // ready for the next launch
+}
+
+template <int G, int W, AttnPasses PASSES>
+__global__ __launch_bounds__(64 * W) void attn_decode_kernel(
+    const f16* q, const f16* kcache, const f16* vcache, int cap, int len, float scale,
+    int splits, float* part, int* counters, f16* out, const f16* knew, const f16* vnew,
+    f16* kcache_w, f16* vcache_w, const float* cosv, const float* sinv, const int* posp) {
+  __shared__ AttnLds<G, W> lds;
+  if (posp) {
+    // decode position in device memory (a captured graph advances it): the
+    // grid covers the cache capacity, the tables hold [cap][half] rows
+    const int pp = min(max(*posp, 0), cap - 1);
+    len = __builtin_amdgcn_readfirstlane(pp + 1);
+    cosv += (long long)pp * (kAttnDim / 2);
+    sinv += (long long)pp * (kAttnDim / 2);
+  }
+  if constexpr (W == 8 && PASSES == kAnyPasses) {
+    // The capacity asks for eight waves, the live length for no more than one
+    // four-wave pass per split: the upper waves end here (a barrier waits only
+    // for waves that have not ended) and the others do what a launch for that
+    // length does.  16/4 heads, capacity 4096: 6.5 us at 256 live positions and
+    // 6.7 at 1024, where eight waves of one pass took 7.7 (two waves a SIMD, and
+    // twice as many to merge in LDS); at 4096 live 7.9.
+    if (len <= kAttnPos * splits) {
+      if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) return;
+      attn_decode<G, 4, kOnePass>(reinterpret_cast<AttnLds<G, 4>&>(lds), q, kcache, vcache, cap, len,
+                                  scale, splits, part, counters, out, knew, vnew, kcache_w, vcache_w,
+                                  cosv, sinv);
+      return;
+    }
+  }
+  attn_decode<G, W, PASSES>(lds, q, kcache, vcache, cap, len, scale, splits, part, counters, out,
+                            knew, vnew, kcache_w, vcache_w, cosv, sinv);
 }
 
 // ---------------------------------------------------------------------------
@@ -572,13 +614,16 @@ hipError_t attn_decode_launch(const void* q, const void* kcache, const void* vca
   const dim3 grid(hkv, splits);
   // longer splits take eight waves: twice the rows on the way to each CU
   const bool wide = len > kAttnPos * splits;
-#define AEXQ_ATTN_W(G, W)                                                                        \
-  hipLaunchKernelGGL((attn_decode_kernel<G, W>), grid, dim3(64 * W), 0, stream, (const f16*)q,  \
+#define AEXQ_ATTN_W(G, W, PASSES)                                                                \
+  hipLaunchKernelGGL((attn_decode_kernel<G, W, PASSES>), grid, dim3(64 * W), 0, stream, (const f16*)q, \
                      (const f16*)kcache, (const f16*)vcache, cap, len, scale, splits, part,      \
                      counters, (f16*)out, (const f16*)knew, (const f16*)vnew, (f16*)kcache,      \
                      (f16*)vcache, cosv, sinv, (const int*)posp)
-#define AEXQ_ATTN(G) \
-  if (wide) AEXQ_ATTN_W(G, 8); else AEXQ_ATTN_W(G, 4)
+#define AEXQ_ATTN(G)                                                        \
+  if (!wide) AEXQ_ATTN_W(G, 4, kOnePass);                                   \
+  else if (posp) AEXQ_ATTN_W(G, 8, kAnyPasses);                             \
+  else if (len <= 2 * kAttnPos * splits) AEXQ_ATTN_W(G, 8, kOnePass);       \
+  else AEXQ_ATTN_W(G, 8, kManyPasses)
   switch (group) {
     case 1: AEXQ_ATTN(1); break;
     case 2: AEXQ_ATTN(2); break;

@@ -114,3 +114,22 @@ def test_positions_that_score_minus_infinity(ctx, length, low):
     ref = _attend(q, kc[:, keep], vc[:, keep], 0.05)
     got = out.cpu().numpy().astype(np.float64)
     assert np.max(np.abs(got - ref)) / np.max(np.abs(ref)) <= TOL
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 4), (16, 8), (16, 4), (8, 1)])
+@pytest.mark.parametrize("live", [1, 64, 65, 200, 1000, 2048])
+def test_device_position_equals_the_launch_for_its_length(ctx, hq, hkv, live):
+    """A device-side position far below the capacity runs the passes that a launch
+    for that length runs (64 positions a split), to the last bit."""
+    print(f"[gpu-case] attention device position {hq}/{hkv} live={live}", flush=True)
+    cap = 9000
+    q, k, v, kc, vc = (torch.as_tensor(a).cuda() for a in _inputs(hq, hkv, cap, live + hq))
+    angle = torch.rand((cap, 64), device="cuda") * 6.28
+    cos, sin = torch.cos(angle), torch.sin(angle)
+    pos = torch.tensor([live - 1], dtype=torch.int32, device="cuda")
+    want, got = torch.zeros_like(q), torch.zeros_like(q)
+    ctx.attention_decode_rope(q, k, v, kc, vc, hq, hkv, D, cap, live, cos[live - 1],
+                              sin[live - 1], 0.088, want)
+    ctx.attention_decode_rope_at(q, k, v, kc, vc, hq, hkv, D, cap, pos, cos, sin, 0.088, got)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
