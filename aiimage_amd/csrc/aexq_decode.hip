@@ -131,7 +131,7 @@ constexpr int kCoherentAux = 16;     // buffer-load cache policy sc1: read at ag
 // One counter per 256-byte line: atomics to one line are serialized where they
 // are performed (about 15 ns each), so the kv heads' counters do not share one.
 constexpr int kAttnCounterStride = 64;
-constexpr int kAttnMaxSplits = 64;   // combine staging in LDS
+constexpr int kAttnMaxSplits = 96;   // combine staging in LDS
 constexpr int kAttnMaxLen = 32768;   // positions a launch takes
 
 // LDS of a workgroup of W waves.
@@ -587,14 +587,22 @@ hipError_t decode_advance_launch(int* position, int* token, const int* argmax, i
 }
 
 // Splits per kv head of a launch over len positions: 64 positions each as long
-// as that keeps the merge short, then longer ones.  Measured (us, heads_q /
-// heads_kv, splits at most 32, 64, 128; with 64 positions a split always):
-// 16/4 at 4096 8.9, 9.5, 9.6 (9.3), at 16384 16.5, 14.6, 18.0 (22.6); 8/1 at
-// 4096 12.1, 14.4, 14.5 (14.5), at 16384 23.0, 18.8, 19.3 (29.1); 32/8 at 8192
-// 14.2, 16.1, 19.0 (18.4); 4/4, whose merge is a quarter, at 4096 7.1, 6.8.
+// as that keeps the merge short, then longer ones, past 4096 positions about a
+// workgroup of eight waves per CU.  Measured (us on rotated caches, so K and V
+// come from HBM; heads_q / heads_kv, splits at most 16, 32, 64; with 64 positions
+// a split always): 16/4 at 4000 10.5, 8.2, 8.9 (8.7), at 16384 21.5, 14.7, 13.3
+// (22.6); 4/4 at 4000 8.4, 6.9, 6.6 (6.6); 32/8 at 8192 14.8, 12.8, 15.8 (18.4);
+// 32/16 at 8192 17.5, 20.5, 24.1 (20.8).  64/16 at 3000 takes 11.9 with 12 splits
+// and 13.9 with 24.  One query head a kv head merges a quarter of that, so on
+// eight kv heads the many short splits stay the better ones for longer: 8/8 at
+// 6000 9.3 against 9.8, at 7000 11.1 against 10.5.
 int attn_splits(int len, int heads_kv, int group) {
-  const int most = len <= 4096 ? (group >= 4 ? 32 : 64) : (heads_kv >= 8 ? 32 : 64);
   const int s = (len + kAttnPos - 1) / kAttnPos;
+  if (group == 1 && heads_kv > 4 && heads_kv <= 8 && len <= kAttnPos * kAttnMaxSplits) return s;
+  const int chip = heads_kv < 256 ? 256 / heads_kv : 1;
+  int most = 64;
+  if (group >= 4 && len <= 4096) most = 32;
+  if (len > (group >= 4 ? 2048 : 4096) && most > chip) most = chip;
   return s < most ? s : most;
 }
 int attn_max_len() { return kAttnMaxLen; }

@@ -56,8 +56,14 @@ def _rotate(x, cos, sin):
     return np.concatenate([a * cos - b * sin, a * sin + b * cos], -1).astype(np.float16)
 
 
-@pytest.mark.parametrize("hq,hkv", [(4, 4), (4, 2), (16, 4), (8, 1), (32, 8)])
-@pytest.mark.parametrize("length", [1, 17, 63, 64, 65, 129, 2047, 2049, 4096, 4097, 8193])
+CASES = [(hq, hkv, length) for hq, hkv in ((4, 4), (4, 2), (16, 4), (8, 1), (32, 8))
+         for length in (1, 17, 63, 64, 65, 129, 2047, 2049, 4096, 4097, 8193)]
+# where the number of splits turns with the kv heads
+CASES += [(hq, hkv, length) for hq, hkv in ((8, 8), (16, 8), (16, 16), (64, 16), (12, 6))
+          for length in (2048, 2049, 4096, 4097, 6144, 6145)]
+
+
+@pytest.mark.parametrize("hq,hkv,length", CASES)
 @pytest.mark.parametrize("form", ["plain", "rope", "rope_at"])
 def test_attention_split_edges(ctx, hq, hkv, length, form):
     print(f"[gpu-case] attention {form} {hq}/{hkv} length={length}", flush=True)
