@@ -1909,8 +1909,7 @@ static aexq_status attn_prepare(aexq_ctx* ctx, const char* op, int heads_q, int 
     return fail(AEXQ_ERR_INVALID_ARGUMENT, op, "length=%d capacity=%d", length, capacity);
   if (length > attn_max_len())
     return fail(AEXQ_ERR_UNSUPPORTED, op, "length=%d (at most %d)", length, attn_max_len());
-  const int splits = attn_splits(length, heads_kv, group);
-  const long long need = (long long)heads_q * splits * attn_part_stride();
+  const long long need = (long long)heads_q * attn_most_splits(length) * attn_part_stride();
   HIP_TRY(op, hipSetDevice(ctx->device));
   aexq_status st = grow_scratch(ctx, (void**)&ctx->attn_part, &ctx->attn_cap,
                                 need * (long long)sizeof(float), op, "attention split partials");

@@ -605,6 +605,13 @@ int attn_splits(int len, int heads_kv, int group) {
   if (len > (group >= 4 ? 2048 : 4096) && most > chip) most = chip;
   return s < most ? s : most;
 }
+// The number turns back at 4097 positions, so the scratch is sized for the most
+// that any length up to len takes: one run at the longest length then covers
+// the shorter ones that a caller captures later.
+int attn_most_splits(int len) {
+  const int s = (len + kAttnPos - 1) / kAttnPos;
+  return s < kAttnMaxSplits ? s : kAttnMaxSplits;
+}
 int attn_max_len() { return kAttnMaxLen; }
 int attn_part_stride() { return kAttnStride; }
 int attn_counter_stride() { return kAttnCounterStride; }

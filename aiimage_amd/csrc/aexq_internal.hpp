@@ -252,9 +252,11 @@ hipError_t embed_q8_launch(const uint32_t* codes, const void* scales, int scale_
 hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, void* vcache,
                           int hq, int hkv, int d, int cap, int pos, const float* cosv,
                           const float* sinv, hipStream_t stream);
-// splits per kv head of a decode attention over `len` positions, and the most
-// positions one launch takes
+// splits per kv head of a decode attention over `len` positions, the most of any
+// length up to `len` (what the scratch holds), and the most positions one launch
+// takes
 int attn_splits(int len, int heads_kv, int group);
+int attn_most_splits(int len);
 int attn_max_len();
 int attn_part_stride();  // fp32 words per (head, split) partial row
 int attn_counter_stride();  // ints between the kv heads' split counters

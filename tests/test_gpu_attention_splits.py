@@ -139,3 +139,31 @@ def test_device_position_equals_the_launch_for_its_length(ctx, hq, hkv, live):
     ctx.attention_decode_rope_at(q, k, v, kc, vc, hq, hkv, D, cap, pos, cos, sin, 0.088, got)
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (8, 8)])
+def test_a_run_at_the_longest_length_covers_captures_of_shorter_ones(aexq, hq, hkv):
+    """The split scratch never has to grow for a shorter length, also where that
+    takes more splits, so its first call may be one under capture."""
+    print(f"[gpu-case] attention capture after a longer run {hq}/{hkv}", flush=True)
+    own = aexq.Context(0)
+    cap, short = 8192, 4096
+    q, _, _, kc, vc = _inputs(hq, hkv, cap, 3)
+    dq, dk, dv = (torch.as_tensor(a).cuda() for a in (q, kc, vc))
+    out = torch.zeros_like(dq)
+    own.attention_decode(dq, dk, dv, hq, hkv, D, cap, cap, 0.088, out)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    own.set_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        own.attention_decode(dq, dk, dv, hq, hkv, D, cap, short, 0.088, out)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = _attend(q, kc[:, :short], vc[:, :short], 0.088)
+        assert np.max(np.abs(out.cpu().numpy() - ref)) / np.max(np.abs(ref)) <= TOL
+    del graph
+    own.close()
