@@ -1534,20 +1534,19 @@ extern "C" aexq_status aexq_plan_check(aexq_ctx* ctx, const aexq_weight* w, cons
     else if (plan.kind == kPlanGemm)
       snprintf(diag, diag_len,
                "kernel=qgemm bits=%d bm=%d swiglu=%d direct=%d fp16_dequant=%d rms_prepass=%d "
-               "tiles=%d grid=%d splitk=%d kstep=%d",
+               "tiles=%d grid=%d waves=%d splitk=%d kstep=%d",
                w->bits, plan.gentry->cfg.bm, (int)plan.gentry->cfg.pair,
                (int)plan.gentry->cfg.direct, (int)plan.gentry->cfg.fd, (int)plan.rms_prepass,
-               plan.p.total_tiles, plan.grid, plan.sk_chunks, plan.gentry->cfg.k128 ? 128 : 64);
+               plan.p.total_tiles, plan.grid, 4 * plan.gentry->cfg.wm, plan.sk_chunks,
+               plan.gentry->cfg.k128 ? 128 : 64);
     else if (plan.kind == kPlanWave)
-      // `splitk` counts the waves a tile's K is split over, inside one launch;
-      // `direct`: fragments straight from memory
+      // `waves`: the K of a tile is split over them, inside one launch
       snprintf(diag, diag_len,
-               "kernel=%s bits=%d mt=%d nt=%d bm=%d swiglu=%d wide=1 direct=1 fp16_dequant=%d "
-               "rms_prepass=%d tiles=%d grid=%d splitk=%d kstep=128",
-               plan.p.m <= 32 ? "qmmk" : "qgemmk", w->bits, plan.kentry->cfg.mt,
-               plan.kentry->cfg.nt, 16 * plan.kentry->cfg.mt, (int)plan.kentry->cfg.pair,
-               (int)plan.kentry->cfg.fd, (int)plan.rms_prepass, plan.p.total_tiles, plan.grid,
-               plan.kentry->cfg.waves);
+               "kernel=wave bits=%d mt=%d nt=%d swiglu=%d ragged=%d fp16_dequant=%d "
+               "rms_prepass=%d tiles=%d grid=%d waves=%d depth=%d splitk=1",
+               w->bits, plan.kentry->cfg.mt, plan.kentry->cfg.nt, (int)plan.kentry->cfg.pair,
+               (int)plan.kentry->cfg.rag, (int)plan.kentry->cfg.fd, (int)plan.rms_prepass,
+               plan.p.total_tiles, plan.grid, plan.kentry->cfg.waves, plan.kdepth);
     else if (plan.kind == kPlanMfma)
       snprintf(diag, diag_len, "kernel=qmm bits=%d mt=%d nt=%d swiglu=%d wide=%d rms_prepass=%d "
                "tiles=%d grid=%d mblock=%d splitk=%d",

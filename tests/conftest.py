@@ -12,6 +12,26 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU and the built HIP library")
 
 
+@pytest.fixture
+def no_wave(monkeypatch):
+    """The wave-split matmul switched off: launches of few tiles take the kernels
+    that those of more tiles take."""
+    monkeypatch.setenv("AEXQ_QMMK_OFF", "1")
+
+
+@pytest.fixture(params=["wave", "other"])
+def wave(request, monkeypatch):
+    """Both sides of that switch: True where the wave-split matmul is on."""
+    if request.param == "other":
+        monkeypatch.setenv("AEXQ_QMMK_OFF", "1")
+    return request.param == "wave"
+
+
+def plan_kernel(plan: str) -> str:
+    """The kernel a plan names, in full."""
+    return plan.split()[0][len("kernel="):]
+
+
 @pytest.fixture(scope="session")
 def orc():
     import oracle

@@ -16,7 +16,7 @@ import sys
 
 import numpy as np
 import pytest
-from conftest import DequantRef, for_plan, q4_reference
+from conftest import DequantRef, for_plan, plan_kernel, q4_reference
 
 torch = pytest.importorskip("torch")
 
@@ -90,7 +90,7 @@ def _weight(ctx, aexq, orc, bits, n, k, seed, group=32, scale_f16=True, code=1):
     (4, 128, False, 515, 2048, 9, True),     # Q4 groups of 128 at M = 9
     (8, 0, False, 257, 576, 32, True),       # K = 9 steps at M = 32
 ])
-def test_gemm_formats(ctx, aexq, orc, bits, group, scale_f16, n, k, m, y32):
+def test_gemm_formats(ctx, aexq, orc, wave, bits, group, scale_f16, n, k, m, y32):
     _announce(f"qgemm q{bits} g={group} f16={scale_f16} n={n} k={k} m={m}")
     from aiimage_amd import synth
     code = 0 if (bits == 4 and m == 129) else 1   # two's complement (reference) vs offset-8
@@ -102,7 +102,8 @@ def test_gemm_formats(ctx, aexq, orc, bits, group, scale_f16, n, k, m, y32):
     xd = aexq.describe(dev(x16), m, k)
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     plan = ctx.plan_check(w, xd, yd)
-    assert plan.startswith("kernel=qgemm"), plan
+    split = wave and k % 128 == 0 and group in (0, 32)   # one launch of the wave-split kernel
+    assert plan_kernel(plan) == ("wave" if split else "qgemm"), plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
     stride = aexq.storage_elements(aexq.LAYOUT_PACK4_LINEAR, m, n)
@@ -118,7 +119,7 @@ def test_gemm_formats(ctx, aexq, orc, bits, group, scale_f16, n, k, m, y32):
 @pytest.mark.parametrize("bits,m,n,k", [(4, 64, 3584, 1024), (4, 150, 1000, 1024),
                                          (8, 96, 640, 1024), (8, 16, 640, 1088),
                                          (4, 20, 1000, 576)])
-def test_gemm_swiglu_rmsnorm(ctx, aexq, orc, bits, m, n, k):
+def test_gemm_swiglu_rmsnorm(ctx, aexq, orc, wave, bits, m, n, k):
     """gate/up with RMSNorm-in (row pre-pass) and SwiGLU-out on the tiled path,
     also at 16 and 20 rows with K not a multiple of 128 (no MFMA block kernel)."""
     _announce(f"qgemm swiglu rms q{bits} m={m} n={n} k={k}")
@@ -133,7 +134,8 @@ def test_gemm_swiglu_rmsnorm(ctx, aexq, orc, bits, m, n, k):
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     kw = dict(rmsnorm=True, rms_gamma=dev(gamma), rms_eps=eps, up=wu)
     plan = ctx.plan_check(wg, xd, yd, **kw)
-    assert plan.startswith("kernel=qgemm") and "rms_prepass=1" in plan and "swiglu=1" in plan, plan
+    assert plan_kernel(plan) == ("wave" if wave and k % 128 == 0 else "qgemm"), plan
+    assert "rms_prepass=1" in plan and "swiglu=1" in plan, plan
     ctx.linear(wg, xd, yd, **kw)
     torch.cuda.synchronize()
     xn = orc.rmsnorm(x16.astype(np.float32), eps, gamma).astype(np.float16).astype(np.float32)
@@ -144,15 +146,18 @@ def test_gemm_swiglu_rmsnorm(ctx, aexq, orc, bits, m, n, k):
     assert normwise(got, ref) <= TOL
 
 
-@pytest.mark.parametrize("path", ["qgemm", "qmm"])
+@pytest.mark.parametrize("path", ["qgemm", "qmm", "wave"])
 @pytest.mark.parametrize("bcast,layout", [(1, "linear"), (3, "linear"), (4, "tiled")])
 def test_gemm_bias_residual(ctx, aexq, orc, monkeypatch, path, bcast, layout):
     """alpha/beta/C per row, per element and per column, with the residual, on
-    the tiled GEMM and (switched off) on the 32-row MFMA blocks."""
+    the tiled GEMM, (switched off) on the 32-row MFMA blocks and on the wave-split
+    kernel."""
     _announce(f"qgemm bias bcast={bcast} layout={layout} path={path}")
     from aiimage_amd import synth
     if path == "qmm":
         monkeypatch.setenv("AEXQ_QGEMM_OFF", "1")
+    if path == "qgemm":
+        monkeypatch.setenv("AEXQ_QMMK_OFF", "1")
     n, k, m = 512, 1024, 70
     w, wf = _weight(ctx, aexq, orc, 8, n, k, 71, scale_f16=False)
     x16 = synth.activations(m, k, 72)
@@ -169,7 +174,7 @@ def test_gemm_bias_residual(ctx, aexq, orc, monkeypatch, path, bcast, layout):
     yd = aexq.describe(y, m, n, lay)
     kw = dict(alpha=0.75, beta=1.5, c=dev(c), broadcast_c=bcast,
               residual=aexq.describe(rd, m, n, lay))
-    assert ctx.plan_check(w, xd, yd, **kw).startswith(f"kernel={path}")
+    assert plan_kernel(ctx.plan_check(w, xd, yd, **kw)) == path
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
     s = orc.gemm_gpu_semantics(x16.astype(np.float32), wf)
@@ -209,7 +214,7 @@ def test_gemm_stacked_copies_batched_x_match_single(ctx, aexq, orc, monkeypatch,
     ys = torch.zeros(copies * m * n, dtype=torch.float16, device="cuda")
     xd = aexq.describe(dev(xs), m, k, batch=copies, batch_stride=m * k)
     yd = aexq.describe(ys, m, n, aexq.LAYOUT_PACK4_LINEAR, batch=copies, batch_stride=m * n)
-    assert ctx.plan_check(st, xd, yd).startswith("kernel=qgemm")
+    assert plan_kernel(ctx.plan_check(st, xd, yd)) == "qgemm"
     ctx.linear(st, xd, yd)
     torch.cuda.synchronize()
     for c in range(copies):
@@ -228,12 +233,13 @@ def test_gemm_stacked_copies_batched_x_match_single(ctx, aexq, orc, monkeypatch,
 ])
 @pytest.mark.parametrize("splitk", ["", "3"])
 @pytest.mark.parametrize("exact", [False, True])
-def test_gemm_group16(ctx, aexq, orc, monkeypatch, scale_f16, n, k, m, swiglu, splitk, exact):
+def test_gemm_group16(ctx, aexq, orc, monkeypatch, wave, scale_f16, n, k, m, swiglu, splitk, exact):
     """Q4 with one scale per 16 codes on the tiled GEMM, in both forms: fp16
     weight tiles (each lane's eight codes of an extent share one scale, one
     MFMA per extent) and the exact one (two MFMAs per 32-code extent, each
     group's product scaled in fp32).  With three forced K chunks the chunks'
-    step counts differ (a tail of the three-step loop, or none)."""
+    step counts differ (a tail of the three-step loop, or none).  Both forms on
+    the wave-split kernel too, where it takes the shape."""
     if splitk:
         monkeypatch.setenv("AEXQ_SPLITK", splitk)
     _announce(f"qgemm group16 f16={scale_f16} n={n} k={k} m={m} swiglu={swiglu} splitk={splitk}")
@@ -248,7 +254,9 @@ def test_gemm_group16(ctx, aexq, orc, monkeypatch, scale_f16, n, k, m, swiglu, s
         wu, uf = _weight(ctx, aexq, orc, 4, n, k, 93 + m, group=16, scale_f16=scale_f16, code=0)
         kw["up"] = wu
     plan = ctx.plan_check(w, xd, yd, **kw)
-    assert plan.startswith("kernel=qgemm") and "direct=1" in plan, plan
+    split = wave and not splitk and k % 128 == 0
+    assert plan_kernel(plan) == ("wave" if split else "qgemm"), plan
+    assert split or "direct=1" in plan, plan
     assert f"fp16_dequant={0 if exact else 1}" in plan, plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
@@ -266,7 +274,7 @@ def test_gemm_group16(ctx, aexq, orc, monkeypatch, scale_f16, n, k, m, swiglu, s
 
 
 @pytest.mark.parametrize("group", [16, 32])
-def test_gemm_q4_extreme_scales_exact(ctx, aexq, orc, group):
+def test_gemm_q4_extreme_scales_exact(ctx, aexq, orc, wave, group):
     """Per-group fp32 scaling keeps the dequantised weight exactly float(q) *
     scale for every fp16 scale: subnormal, large and above 4096 (where q * s
     would overflow an fp16 product) among the groups -- the fp32-output bar
@@ -289,7 +297,8 @@ def test_gemm_q4_extreme_scales_exact(ctx, aexq, orc, group):
     xd = aexq.describe(dev(x16), m, k)
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     plan = ctx.plan_check(w, xd, yd, exact=True)
-    assert "direct=1" in plan and "fp16_dequant=0" in plan, plan
+    assert plan_kernel(plan) == ("wave" if wave else "qgemm") and "fp16_dequant=0" in plan, plan
+    assert wave or "direct=1" in plan, plan
     ctx.linear(w, xd, yd, exact=True)
     torch.cuda.synchronize()
     ref = orc.gemm_gpu_semantics(x16.astype(np.float32), wf)
@@ -297,7 +306,7 @@ def test_gemm_q4_extreme_scales_exact(ctx, aexq, orc, group):
 
 
 @pytest.mark.parametrize("big", [8000.0, 9000.0, float("inf")])
-def test_gemm_fp16_dequant_needs_finite_products(ctx, aexq, orc, big):
+def test_gemm_fp16_dequant_needs_finite_products(ctx, aexq, orc, wave, big):
     """The fp16 weight tile is chosen only when 8 |s| fits fp16 for every scale
     of the weight: a weight with one fp32 scale of 9000 (q * s up to 72000)
     takes the exact form by itself and stays within the fp32 bar; 8000 (64000,
@@ -318,6 +327,7 @@ def test_gemm_fp16_dequant_needs_finite_products(ctx, aexq, orc, big):
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     plan = ctx.plan_check(w, xd, yd)
     want_fd = big < 65504.0 / 8
+    assert plan_kernel(plan) == ("wave" if wave else "qgemm"), plan
     assert f"fp16_dequant={int(want_fd)}" in plan, plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
@@ -374,7 +384,7 @@ def test_gemm_direct_pairs(ctx, aexq, orc, bits, group, scale_f16, m):
     y = aexq.new_activation(m, n, torch.float32, aexq.LAYOUT_PACK4_LINEAR)
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     plan = ctx.plan_check(wg, xd, yd, up=wu)
-    assert plan.startswith("kernel=qgemm") and "direct=1" in plan, plan
+    assert plan_kernel(plan) == "qgemm" and "direct=1" in plan, plan
     ctx.linear(wg, xd, yd, up=wu)
     torch.cuda.synchronize()
     g = orc.gemm_gpu_semantics(x16.astype(np.float32), for_plan(gf, plan))

@@ -92,7 +92,7 @@ def test_eight_wave_tiles(ctx, aexq, orc, bits, group, f16, m, n, k, epi, cols):
         bias = synth.activations(1, n, 5).astype(np.float32).reshape(-1)
         kw.update(alpha=0.75, beta=1.25, c=dev(bias), broadcast_c=4)
     plan = dict(t.split("=") for t in ctx.plan_check(w, xd, yd, **kw).split())
-    assert plan["kernel"] == "qgemm" and plan["bm"] == "128" and plan["splitk"] == "1", plan
+    assert plan["kernel"] == "qgemm" and plan["waves"] == "8" and plan["splitk"] == "1", plan
     assert int(plan["tiles"]) == -(-(n if epi == "heads" else stride) // cols), plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()

@@ -11,7 +11,7 @@ import sys
 
 import numpy as np
 import pytest
-from conftest import for_plan, q4_reference
+from conftest import for_plan, plan_kernel, q4_reference
 
 torch = pytest.importorskip("torch")
 
@@ -91,6 +91,8 @@ def test_qkv_group_head_packed_m1_rmsnorm(ctx, aexq, orc):
     (20, 1024, False, "qmm"),     # MFMA 32-row blocks
     (70, 1024, True, "qgemm"),    # tiled GEMM, two 64-row tiles
     (40, 1024, True, "qmm"),      # MFMA over two row blocks (tiled GEMM switched off)
+    (20, 1024, False, "wave"),    # wave-split, exact products
+    (70, 1024, True, "wave"),     # wave-split, fp16 weight tiles
     (3, 40, True, "generic"),     # K not a whole 32-code chunk: the generic kernel
 ])
 def test_head_packed_output_families(ctx, aexq, orc, monkeypatch, m, k, y32, kernel):
@@ -100,6 +102,8 @@ def test_head_packed_output_families(ctx, aexq, orc, monkeypatch, m, k, y32, ker
     from aiimage_amd import synth
     if kernel == "qmm" and m > 32:
         monkeypatch.setenv("AEXQ_QGEMM_OFF", "1")
+    if kernel != "wave":
+        monkeypatch.setenv("AEXQ_QMMK_OFF", "1")
     heads, hd = 6, 64
     n = heads * hd
     if k % 32:
@@ -115,7 +119,7 @@ def test_head_packed_output_families(ctx, aexq, orc, monkeypatch, m, k, y32, ker
     xd = aexq.describe(dev(x16), m, k)
     yd = aexq.describe(y, m, n, aexq.LAYOUT_HEAD_PACKED, head_dim=hd)
     plan = ctx.plan_check(w, xd, yd)
-    assert plan.startswith(f"kernel={kernel}"), plan
+    assert plan_kernel(plan) == kernel, plan
     ctx.linear(w, xd, yd, alpha=0.5)
     torch.cuda.synchronize()
     got = y.cpu().numpy().astype(np.float64)

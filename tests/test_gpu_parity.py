@@ -9,6 +9,7 @@ import sys
 
 import numpy as np
 import pytest
+from conftest import plan_kernel
 
 torch = pytest.importorskip("torch")
 
@@ -627,33 +628,33 @@ def _mm_case(ctx, aexq, orc, fmt, n, k, m, seed, group=32, code=1, scale_f16=Tru
 @pytest.mark.parametrize("fmt,n,k,m", [(8, 3584, 1024, 16), (8, 1024, 2048, 64), (8, 1024, 1024, 512),
                                        (4, 3584, 1024, 16), (4, 1024, 3584, 64), (4, 2048, 1024, 512),
                                        (4, 512, 1024, 5), (8, 256, 384, 31)])
-def test_small_m_mfma_config4(ctx, aexq, orc, fmt, n, k, m):
+def test_small_m_mfma_config4(ctx, aexq, orc, wave, fmt, n, k, m):
     """Batched decode / short prefill shapes on the MFMA path against the float64 oracle."""
     _announce(f"mfma q{fmt} n={n} k={k} m={m}")
     got, wf, x16, plan = _mm_case(ctx, aexq, orc, fmt, n, k, m, seed=n + k + m)
-    # M > 32: the tiled GEMM; M <= 32: one MFMA launch of 16- or 32-row blocks
-    assert plan.startswith("kernel=qgemm" if m > 32 else "kernel=qmm"), plan
+    # switched off: M > 32 the tiled GEMM; M <= 32 one MFMA launch of 16- or 32-row blocks
+    assert plan_kernel(plan) == ("wave" if wave else "qgemm" if m > 32 else "qmm"), plan
     ref = orc.gemm_gpu_semantics(x16.astype(np.float32), wf)
     assert normwise(got, ref) <= TOL
 
 
 @pytest.mark.parametrize("group,scale_f16,code", [(16, False, 0), (16, True, 0), (32, False, 0)])
-def test_small_m_mfma_reference_q4_formats(ctx, aexq, orc, group, scale_f16, code):
+def test_small_m_mfma_reference_q4_formats(ctx, aexq, orc, wave, group, scale_f16, code):
     """The reference's shipping Q4 (two's complement, group 16, fp32 scales) and its
     neighbours at M > 1, fp32 output for a tight bar."""
     _announce(f"mfma q4 group={group} f16={scale_f16}")
     got, wf, x16, plan = _mm_case(ctx, aexq, orc, 4, 1024, 1024, 12, seed=40 + group,
                                   group=group, code=code, scale_f16=scale_f16,
                                   ydtype=torch.float32)
-    assert plan.startswith("kernel=qmm"), plan
+    assert plan_kernel(plan) == ("wave" if wave else "qmm"), plan
     ref = orc.gemm_gpu_semantics(x16.astype(np.float32), wf)
     assert normwise(got, ref) <= 1e-5
 
 
 @pytest.mark.parametrize("prepass", [False, True])
-def test_small_m_mfma_swiglu_rmsnorm(ctx, aexq, orc, monkeypatch, prepass):
+def test_small_m_mfma_swiglu_rmsnorm(ctx, aexq, orc, monkeypatch, wave, prepass):
     """M=20 gate/up with RMSNorm-in and SwiGLU-out on the MFMA path: inside the
-    wide kernel (one item per workgroup) or as the row pre-pass."""
+    kernel (the wide one: one item per workgroup) or as the row pre-pass."""
     _announce(f"mfma swiglu rmsnorm m=20 prepass={prepass}")
     if prepass:
         monkeypatch.setenv("AEXQ_RMS_PREPASS", "1")
@@ -668,7 +669,8 @@ def test_small_m_mfma_swiglu_rmsnorm(ctx, aexq, orc, monkeypatch, prepass):
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     kw = dict(rmsnorm=True, rms_gamma=dev(gamma), rms_eps=eps, up=wu)
     plan = ctx.plan_check(wg, xd, yd, **kw)
-    assert plan.startswith("kernel=qmm") and f"rms_prepass={int(prepass)}" in plan, plan
+    assert plan_kernel(plan) == ("wave" if wave else "qmm"), plan
+    assert f"rms_prepass={int(prepass)}" in plan, plan
     ctx.linear(wg, xd, yd, **kw)
     torch.cuda.synchronize()
     xn = orc.rmsnorm(x16.astype(np.float32), eps, gamma).astype(np.float16).astype(np.float32)
@@ -699,7 +701,7 @@ def test_small_m_mfma_row_blocks_bias_residual(ctx, aexq, orc, monkeypatch, bcas
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     kw = dict(alpha=0.75, beta=1.5, c=dev(c), broadcast_c=bcast,
               residual=aexq.describe(rd, m, n, aexq.LAYOUT_PACK4_LINEAR))
-    assert ctx.plan_check(w, xd, yd, **kw).startswith("kernel=qmm")
+    assert plan_kernel(ctx.plan_check(w, xd, yd, **kw)) == "qmm"
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
     s = orc.gemm_gpu_semantics(x16.astype(np.float32), orc.dequant_q8(words, scales, n, k))

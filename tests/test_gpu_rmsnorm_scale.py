@@ -25,6 +25,7 @@ import sys
 
 import numpy as np
 import pytest
+from conftest import plan_kernel
 
 torch = pytest.importorskip("torch")
 
@@ -223,7 +224,7 @@ def test_streaming_m5(ctx, aexq, orc, name, scale, gval):
 
 @pytest.mark.parametrize("prepass", [False, True])
 @pytest.mark.parametrize("name,scale,gval", SCALES)
-def test_mfma_m16(ctx, aexq, orc, monkeypatch, prepass, name, scale, gval):
+def test_mfma_m16(ctx, aexq, orc, monkeypatch, wave, prepass, name, scale, gval):
     _announce(f"rms mfma m=16 prepass={prepass} {name}")
     if prepass:
         monkeypatch.setenv("AEXQ_RMS_PREPASS", "1")
@@ -235,7 +236,7 @@ def test_mfma_m16(ctx, aexq, orc, monkeypatch, prepass, name, scale, gval):
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     kw = dict(rmsnorm=True, rms_gamma=dev(gamma), rms_eps=EPS)
     plan = ctx.plan_check(w, xd, yd, **kw)
-    assert plan.startswith("kernel=qmm"), plan
+    assert plan_kernel(plan) == ("wave" if wave else "qmm"), plan
     assert ("rms_prepass=1" in plan) == prepass, plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()

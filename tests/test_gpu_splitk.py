@@ -13,7 +13,7 @@ import sys
 
 import numpy as np
 import pytest
-from conftest import for_plan, q4_reference
+from conftest import for_plan, plan_kernel, q4_reference
 
 torch = pytest.importorskip("torch")
 
@@ -101,7 +101,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("bits,scale_f16,n,k,m,y32,kernel", CASES)
-def test_split_matches_oracle(ctx, aexq, orc, monkeypatch, bits, scale_f16, n, k, m, y32, kernel):
+def test_split_matches_oracle(ctx, aexq, orc, monkeypatch, no_wave, bits, scale_f16, n, k, m, y32, kernel):
     _announce(f"splitk q{bits} f16={scale_f16} n={n} k={k} m={m} y32={y32} {kernel}")
     from aiimage_amd import synth
     w, wf = _weight(ctx, aexq, orc, bits, n, k, n + k + m, scale_f16=scale_f16)
@@ -112,7 +112,7 @@ def test_split_matches_oracle(ctx, aexq, orc, monkeypatch, bits, scale_f16, n, k
     y = aexq.new_activation(m, n, ydt, lay)
     yd = aexq.describe(y, m, n, lay)
     plan = ctx.plan_check(w, xd, yd)
-    assert plan.startswith(f"kernel={kernel}") and _splitk(plan) > 1, plan
+    assert plan_kernel(plan) == kernel and _splitk(plan) > 1, plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
     stride = aexq.storage_elements(lay, m, n)
@@ -158,7 +158,7 @@ def test_split_narrow_kernel(ctx, aexq, orc, monkeypatch, bits, group, n, k, m, 
                          code=0)
         kw = dict(up=wu)
     plan = ctx.plan_check(w, xd, yd, **kw)
-    assert plan.startswith("kernel=qmm") and "wide=0" in plan and _splitk(plan) > 1, plan
+    assert plan_kernel(plan) == "qmm" and "wide=0" in plan and _splitk(plan) > 1, plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
     g = orc.gemm_gpu_semantics(x16.astype(np.float32), for_plan(wf, plan))
@@ -176,9 +176,9 @@ def test_split_narrow_kernel(ctx, aexq, orc, monkeypatch, bits, group, n, k, m, 
     (False, 32, True, True),     # gate/up pair at M = 32 with RMSNorm-in in the kernel
     (True, 9, False, True),      # fp16 scales, RMSNorm-in
 ])
-def test_wide_kernel_group16(ctx, aexq, orc, scale_f16, m, pair, rms):
-    """Group-16 Q4 on the wide kernel: two MFMAs per 32-code extent, each
-    group's product scaled in fp32 (exact float(q) * scale)."""
+def test_wide_kernel_group16(ctx, aexq, orc, wave, scale_f16, m, pair, rms):
+    """Group-16 Q4 on the wide kernel, and on the wave-split one: two MFMAs per
+    32-code extent, each group's product scaled in fp32 (exact float(q) * scale)."""
     _announce(f"wide group16 f16={scale_f16} m={m} pair={pair} rms={rms}")
     from aiimage_amd import synth
     n, k, eps = 1024, 2048, 1e-6
@@ -195,7 +195,8 @@ def test_wide_kernel_group16(ctx, aexq, orc, scale_f16, m, pair, rms):
     xd = aexq.describe(dev(x16), m, k)
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     plan = ctx.plan_check(w, xd, yd, **kw)
-    assert plan.startswith("kernel=qmm") and "wide=1" in plan, plan
+    assert plan_kernel(plan) == ("wave" if wave else "qmm"), plan
+    assert wave or "wide=1" in plan, plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
     xr = x16.astype(np.float32)
@@ -231,7 +232,7 @@ def test_forced_chunk_counts(ctx, aexq, orc, monkeypatch, chunks, kernel, m):
     steps = k // (256 if kernel == "qmm" else _kstep(plan))
     want = min(int(chunks), steps)
     cs = -(-steps // want)
-    assert plan.startswith(f"kernel={kernel}") and _splitk(plan) == -(-steps // cs), plan
+    assert plan_kernel(plan) == kernel and _splitk(plan) == -(-steps // cs), plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
     ref = orc.gemm_gpu_semantics(x16.astype(np.float32), for_plan(wf, plan))
@@ -239,9 +240,9 @@ def test_forced_chunk_counts(ctx, aexq, orc, monkeypatch, chunks, kernel, m):
 
 
 @pytest.mark.parametrize("bits,m", [(4, 16), (8, 32), (4, 64), (8, 200)])
-def test_split_swiglu_rmsnorm(ctx, aexq, orc, bits, m):
+def test_split_swiglu_rmsnorm(ctx, aexq, orc, wave, bits, m):
     """gate/up with RMSNorm-in and SwiGLU-out: both halves' partials summed, then
-    silu(gate) * up in the fix-up."""
+    silu(gate) * up in the fix-up (the wave-split kernel: the waves' in LDS)."""
     _announce(f"splitk swiglu q{bits} m={m}")
     from aiimage_amd import synth
     n, k, eps = 1024, 2048, 1e-6
@@ -254,7 +255,7 @@ def test_split_swiglu_rmsnorm(ctx, aexq, orc, bits, m):
     yd = aexq.describe(y, m, n, aexq.LAYOUT_PACK4_LINEAR)
     kw = dict(rmsnorm=True, rms_gamma=dev(gamma), rms_eps=eps, up=wu)
     plan = ctx.plan_check(wg, xd, yd, **kw)
-    assert "swiglu=1" in plan and _splitk(plan) > 1, plan
+    assert "swiglu=1" in plan and (plan_kernel(plan) == "wave" if wave else _splitk(plan) > 1), plan
     ctx.linear(wg, xd, yd, **kw)
     torch.cuda.synchronize()
     xn = orc.rmsnorm(x16.astype(np.float32), eps, gamma).astype(np.float16).astype(np.float32)
@@ -267,9 +268,9 @@ def test_split_swiglu_rmsnorm(ctx, aexq, orc, bits, m):
 
 @pytest.mark.parametrize("bcast,layout,m", [(1, "linear", 24), (3, "linear", 70), (4, "tiled", 16),
                                             (4, "tiled", 300)])
-def test_split_bias_residual(ctx, aexq, orc, bcast, layout, m):
+def test_split_bias_residual(ctx, aexq, orc, wave, bcast, layout, m):
     """alpha/beta/C (per row, per element, per column) and the residual run in
-    the fix-up, in both Gemm bias forms."""
+    the fix-up (or the wave-split kernel's epilogue), in both Gemm bias forms."""
     _announce(f"splitk bias bcast={bcast} layout={layout} m={m}")
     from aiimage_amd import synth
     n, k = 512, 2048
@@ -287,7 +288,8 @@ def test_split_bias_residual(ctx, aexq, orc, bcast, layout, m):
     yd = aexq.describe(y, m, n, lay)
     kw = dict(alpha=0.75, beta=1.5, c=dev(c), broadcast_c=bcast,
               residual=aexq.describe(dev(rbuf), m, n, lay))
-    assert _splitk(ctx.plan_check(w, xd, yd, **kw)) > 1
+    plan = ctx.plan_check(w, xd, yd, **kw)
+    assert plan_kernel(plan) == "wave" if wave else _splitk(plan) > 1, plan
     ctx.linear(w, xd, yd, **kw)
     torch.cuda.synchronize()
     s = orc.gemm_gpu_semantics(x16.astype(np.float32), wf)
@@ -303,7 +305,7 @@ def test_split_bias_residual(ctx, aexq, orc, bcast, layout, m):
 
 
 @pytest.mark.parametrize("m", [16, 40])
-def test_split_grouped_head_packed(ctx, aexq, orc, m):
+def test_split_grouped_head_packed(ctx, aexq, orc, wave, m):
     """A q/k/v group (three matrices' partial planes side by side) into
     attention head-packed outputs."""
     _announce(f"splitk qkv head-packed m={m}")
@@ -320,6 +322,7 @@ def test_split_grouped_head_packed(ctx, aexq, orc, m):
         ys.append(y)
         yds.append(aexq.describe(y, m, n, aexq.LAYOUT_HEAD_PACKED, head_dim=hd))
         plan = ctx.plan_check(w, xd, yds[-1])
+        assert plan_kernel(plan) == "wave" if wave else _splitk(plan) > 1, plan
         refs.append(orc.gemm_gpu_semantics(x16.astype(np.float32), for_plan(wf, plan)))
     ctx.linear_group(ws, xd, yds)
     torch.cuda.synchronize()
@@ -340,11 +343,11 @@ def test_batched_stack_keeps_whole_tiles(ctx, aexq, orc):
     plan = ctx.plan_check(st, aexq.describe(x, m, k),
                           aexq.describe(ys, m, n, aexq.LAYOUT_PACK4_LINEAR, batch=copies,
                                         batch_stride=m * n))
-    assert _splitk(plan) == 1, plan
+    assert plan_kernel(plan) == "qmm" and _splitk(plan) == 1, plan
     st.release()
 
 
-def test_split_graph_replays_match_eager(ctx, aexq, orc):
+def test_split_graph_replays_match_eager(ctx, aexq, orc, wave):
     """A layer's split launches (q/k/v group, gate/up pair, o_proj, down at M = 16
     and 64) captured in a HIP graph: every replay, with eager work between
     replays, equals the eager result bit for bit (the partial planes are fully
@@ -372,7 +375,8 @@ def test_split_graph_replays_match_eager(ctx, aexq, orc):
             ctx.linear(ws["o_proj"], xd[2048], yd["o_proj"])
             ctx.linear(ws["down_proj"], xd[3584], yd["down_proj"])
 
-        assert _splitk(ctx.plan_check(ws["down_proj"], xd[3584], yd["down_proj"])) > 1
+        plan = ctx.plan_check(ws["down_proj"], xd[3584], yd["down_proj"])
+        assert plan_kernel(plan) == "wave" if wave else _splitk(plan) > 1, plan
         step()
         torch.cuda.synchronize()
         eager = {k: v.clone() for k, v in ys.items()}
@@ -406,9 +410,9 @@ def test_split_graph_replays_match_eager(ctx, aexq, orc):
     (4, 16, False, False), (4, 9, True, False), (8, 24, False, False), (8, 32, True, False),
     (4, 16, False, True),   # a q/k/v group sharing one normalised input
 ])
-def test_rmsnorm_in_kernel(ctx, aexq, orc, monkeypatch, bits, m, pair, group):
-    """RMSNorm-in inside the wide kernel (launches with one item per workgroup):
-    no pre-pass launch, the oracle's RMSNorm -> fp16 -> Gemm within the fp16 bar,
+def test_rmsnorm_in_kernel(ctx, aexq, orc, monkeypatch, wave, bits, m, pair, group):
+    """RMSNorm-in inside the wide kernel (launches with one item per workgroup)
+    and inside the wave-split one: no pre-pass launch, the oracle's RMSNorm -> fp16 -> Gemm within the fp16 bar,
     and the pre-pass path's result within one fp16 rounding of the inputs."""
     _announce(f"rmsnorm in-kernel q{bits} m={m} pair={pair} group={group}")
     from aiimage_amd import synth
@@ -438,7 +442,8 @@ def test_rmsnorm_in_kernel(ctx, aexq, orc, monkeypatch, bits, m, pair, group):
         return ys, ctx.plan_check(ws[0], xd, yds[0], **kw)
 
     ys, plan = run()
-    assert "wide=1" in plan and "rms_prepass=0" in plan, plan
+    assert plan_kernel(plan) == ("wave" if wave else "qmm") and "rms_prepass=0" in plan, plan
+    assert wave or "wide=1" in plan, plan
     monkeypatch.setenv("AEXQ_RMS_PREPASS", "1")
     ys_pre, plan_pre = run()
     assert "rms_prepass=1" in plan_pre, plan_pre

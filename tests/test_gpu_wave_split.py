@@ -12,7 +12,7 @@ import sys
 
 import numpy as np
 import pytest
-from conftest import for_plan, q4_reference
+from conftest import for_plan, plan_kernel, q4_reference
 
 torch = pytest.importorskip("torch")
 
@@ -72,26 +72,26 @@ def _weight(ctx, aexq, orc, fmt, n, k, seed, poke=None):
 # (fmt, m, n, k, epilogue, expected kernel)
 CASES = [
     # row tiles: 16, 32 and 64 rows and one past; one 128-wide slice and many
-    ("q4h", 2, 16, 128, "plain", "qmmk"), ("q8h", 16, 33, 256, "plain", "qmmk"),
-    ("q4g16s", 17, 1000, 1024, "plain", "qmmk"), ("q8s", 32, 5137, 512, "plain", "qmmk"),
-    ("q4h", 32, 11000, 1024, "plain", "qmmk"), ("q4s", 16, 5200, 1152, "plain", "qmmk"),
-    ("q8h", 33, 1001, 1024, "plain", "qgemmk"), ("q4h", 64, 1024, 3584, "plain", "qgemmk"),
-    ("q4g16h", 65, 515, 512, "plain", "qgemmk"), ("q4s", 97, 3000, 640, "plain", "qgemmk"),
-    ("q8s", 130, 4100, 1024, "plain", "qgemmk"), ("q4g16s", 257, 4096, 1024, "plain", "qgemmk"),
-    ("q4h", 500, 1024, 2048, "residual", "qgemmk"), ("q8h", 300, 3072, 1024, "residual", "qgemmk"),
+    ("q4h", 2, 16, 128, "plain", "wave"), ("q8h", 16, 33, 256, "plain", "wave"),
+    ("q4g16s", 17, 1000, 1024, "plain", "wave"), ("q8s", 32, 5137, 512, "plain", "wave"),
+    ("q4h", 32, 11000, 1024, "plain", "wave"), ("q4s", 16, 5200, 1152, "plain", "wave"),
+    ("q8h", 33, 1001, 1024, "plain", "wave"), ("q4h", 64, 1024, 3584, "plain", "wave"),
+    ("q4g16h", 65, 515, 512, "plain", "wave"), ("q4s", 97, 3000, 640, "plain", "wave"),
+    ("q8s", 130, 4100, 1024, "plain", "wave"), ("q4g16s", 257, 4096, 1024, "plain", "wave"),
+    ("q4h", 500, 1024, 2048, "residual", "wave"), ("q8h", 300, 3072, 1024, "residual", "wave"),
     # SwiGLU pairs; RMSNorm-in: one slice a wave, whole rows in the ring, past it
-    ("q4h", 5, 3584, 1024, "swiglu", "qmmk"), ("q8h", 31, 3000, 2048, "swiglu", "qmmk"),
-    ("q4g16h", 32, 5200, 1024, "swiglu", "qmmk"), ("q8s", 16, 130, 4096, "rms", "qmmk"),
-    ("q4g16s", 3, 257, 3072, "rms", "qmmk"), ("q4s", 30, 640, 2048, "rms", "qmmk"),
-    ("q4h", 29, 5201, 2048, "rms", "qmmk"), ("q4h", 16, 520, 1024, "rms-nogamma", "qmmk"),
-    ("q4s", 64, 200, 1024, "rms", "qgemmk"), ("q8h", 100, 1024, 512, "swiglu", "qgemmk"),
+    ("q4h", 5, 3584, 1024, "swiglu", "wave"), ("q8h", 31, 3000, 2048, "swiglu", "wave"),
+    ("q4g16h", 32, 5200, 1024, "swiglu", "wave"), ("q8s", 16, 130, 4096, "rms", "wave"),
+    ("q4g16s", 3, 257, 3072, "rms", "wave"), ("q4s", 30, 640, 2048, "rms", "wave"),
+    ("q4h", 29, 5201, 2048, "rms", "wave"), ("q4h", 16, 520, 1024, "rms-nogamma", "wave"),
+    ("q4s", 64, 200, 1024, "rms", "wave"), ("q8h", 100, 1024, 512, "swiglu", "wave"),
     # K of 16-code halves of a chunk, of odd scale rows, of less than a slice
-    ("q8s", 77, 1001, 1008, "plain", "qgemmk"), ("q8h", 9, 50, 16, "plain", "qmmk"),
-    ("q4g16h", 1, 97, 1040, "plain", "qmmk"), ("q4g16h", 200, 333, 336, "residual", "qgemmk"),
-    ("q4g16s", 5, 101, 48, "plain", "qmmk"), ("q4h", 19, 345, 1120, "plain", "qmmk"),
-    ("q4h", 300, 900, 160, "plain", "qgemmk"), ("q4s", 12, 64, 32, "plain", "qmmk"),
-    ("q4g16s", 40, 70, 2000, "rms", "qgemmk"), ("q4g16h", 700, 640, 208, "rms", "qgemmk"),
-    ("q8h", 33, 129, 4080, "rms", "qgemmk"),
+    ("q8s", 77, 1001, 1008, "plain", "wave"), ("q8h", 9, 50, 16, "plain", "wave"),
+    ("q4g16h", 1, 97, 1040, "plain", "wave"), ("q4g16h", 200, 333, 336, "residual", "wave"),
+    ("q4g16s", 5, 101, 48, "plain", "wave"), ("q4h", 19, 345, 1120, "plain", "wave"),
+    ("q4h", 300, 900, 160, "plain", "wave"), ("q4s", 12, 64, 32, "plain", "wave"),
+    ("q4g16s", 40, 70, 2000, "rms", "wave"), ("q4g16h", 700, 640, 208, "rms", "wave"),
+    ("q8h", 33, 129, 4080, "rms", "wave"),
 ]
 
 
@@ -125,7 +125,7 @@ def test_wave_split_against_oracle(ctx, aexq, orc, fmt, m, n, k, epi, kernel):
         y.fill_(7.0)   # the padding lanes must be written
         yd = aexq.describe(y, m, n, lay)
         plan = ctx.plan_check(w, xd, yd, **kw)
-        assert plan.startswith(f"kernel={kernel} "), plan
+        assert plan_kernel(plan) == kernel, plan
         ctx.linear(w, xd, yd, **kw)
         ys.append(y)
     torch.cuda.synchronize()
@@ -156,7 +156,7 @@ def test_wave_split_stack_equals_single(ctx, aexq, orc, fmt, m, k):
     ys = aexq.new_activation(m, n, torch.float32, lay, batch=copies)
     xd = aexq.describe(xs, m, k, batch=copies, batch_stride=m * k)
     yd = aexq.describe(ys, m, n, lay, batch=copies, batch_stride=m * n)
-    assert "splitk=8" in ctx.plan_check(st, xd, yd)
+    assert plan_kernel(ctx.plan_check(st, xd, yd)) == "wave"
     ctx.linear(st, xd, yd)
     for c in range(copies):
         y = aexq.new_activation(m, n, torch.float32, lay)
@@ -180,7 +180,7 @@ def test_ragged_k_keeps_to_its_row(ctx, aexq, orc, fmt):
     y = aexq.new_activation(m, n, torch.float32, aexq.LAYOUT_LINEAR)
     xd, yd = aexq.describe(dev(x16), m, k), aexq.describe(y, m, n)
     plan = ctx.plan_check(w, xd, yd)
-    assert plan.startswith("kernel=qmmk "), plan
+    assert plan.startswith("kernel=wave "), plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
     got = y.cpu().numpy().reshape(m, n)
@@ -206,7 +206,7 @@ def test_infinite_activation_keeps_its_sign(ctx, aexq, orc, fmt, m, k):
     y = aexq.new_activation(m, n, torch.float32, aexq.LAYOUT_LINEAR)
     xd, yd = aexq.describe(dev(x16), m, k), aexq.describe(y, m, n)
     plan = ctx.plan_check(w, xd, yd)
-    assert plan.startswith("kernel=qmmk "), plan
+    assert plan.startswith("kernel=wave "), plan
     ctx.linear(w, xd, yd)
     torch.cuda.synchronize()
     got = y.cpu().numpy().reshape(m, n)
@@ -236,10 +236,10 @@ def test_rows_too_far_apart_for_its_offsets(ctx, aexq, orc):
         yd = rows_of(y, n, rs)
         return ctx.plan_check(w, rows_of(x, k, xs), yd, residual=yd).split()[0]
 
-    assert kernel(k, n) == "kernel=qmmk"
-    assert kernel((1 << 23) - 8, (1 << 22) - 8) == "kernel=qmmk"
-    assert kernel(1 << 23, n) != "kernel=qmmk"
-    assert kernel(k, 1 << 22) != "kernel=qmmk"
+    assert kernel(k, n) == "kernel=wave"
+    assert kernel((1 << 23) - 8, (1 << 22) - 8) == "kernel=wave"
+    assert kernel(1 << 23, n) != "kernel=wave"
+    assert kernel(k, 1 << 22) != "kernel=wave"
 
 
 def test_other_kernels_where_they_stay(ctx, aexq, orc):
