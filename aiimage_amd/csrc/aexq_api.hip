@@ -1146,7 +1146,8 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       t16 += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + 15) / 16 * w0->batch;
     QmmkConfig kc{fmt, fmt == kQ8 ? 0 : w0->block, w0->scale_dtype == AEXQ_DTYPE_F16,
                   !rag && M > 32 && fd, 1, 1, 8, swiglu, fused, rag};
-    if (!qmmk_pick(M, t16, fmt == kQ8, swiglu, rag, &kc.mt, &kc.nt, &kc.waves)) return;
+    const QmmkShape shape{M, K, t16, fmt, kc.g, kc.fd, swiglu, fused, rag, ctx->cus};
+    if (!qmmk_pick(shape, &kc.mt, &kc.nt, &kc.waves)) return;
     const char* env = getenv("AEXQ_QMMK_TILE");  // tuning: "mt:nt:waves"
     if (env && sscanf(env, "%d:%d:%d", &kc.mt, &kc.nt, &kc.waves) != 3) return;
     const QmmkEntry* e = qmmk_find(kc);

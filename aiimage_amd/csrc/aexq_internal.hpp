@@ -202,9 +202,17 @@ const QmmkEntry* qmmk_table_q8(int* count);
 const QmmkEntry* qmmk_table_q4(int* count);     // exact products
 const QmmkEntry* qmmk_table_q4_fd(int* count);  // fp16 weight tiles
 const QmmkEntry* qmmk_find(const QmmkConfig& cfg);
-// The tile and wave count for m rows by t16 16-row weight blocks (over every
-// matrix and copy); false: another kernel is the better one.
-bool qmmk_pick(int m, long long t16, bool q8, bool pair, bool rag, int* mt, int* nt, int* waves);
+// A launch of the wave-split matmul: m rows by t16 16-row weight blocks (over
+// every matrix and copy), K long, on a part of `cus` CUs.
+struct QmmkShape {
+  int m, k;
+  long long t16;
+  int fmt, g;
+  bool fd, pair, rms, rag;  // as in QmmkConfig
+  int cus;
+};
+// Its tile and wave count; false: another kernel is the better one.
+bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves);
 // LDS slots per wave of a launch of `wgs` workgroups on `cus` CUs
 int qmmk_depth(const QmmkEntry* e, int k, long long wgs, int cus);
 hipError_t qmmk_launch(const QmmkEntry* e, const QmvParams& p, int depth, hipStream_t stream);

@@ -81,7 +81,8 @@ CASES = [
     ("q4h", 500, 1024, 2048, "residual", "wave"), ("q8h", 300, 3072, 1024, "residual", "wave"),
     # SwiGLU pairs; RMSNorm-in: one slice a wave, whole rows in the ring, past it
     ("q4h", 5, 3584, 1024, "swiglu", "wave"), ("q8h", 31, 3000, 2048, "swiglu", "wave"),
-    ("q4g16h", 32, 5200, 1024, "swiglu", "wave"), ("q8s", 16, 130, 4096, "rms", "wave"),
+    ("q4g16h", 32, 4090, 1024, "swiglu", "wave"), ("q8s", 16, 130, 4096, "rms", "wave"),
+    ("q4h", 32, 5200, 1024, "swiglu", "wave"),
     ("q4g16s", 3, 257, 3072, "rms", "wave"), ("q4s", 30, 640, 2048, "rms", "wave"),
     ("q4h", 29, 5201, 2048, "rms", "wave"), ("q4h", 16, 520, 1024, "rms-nogamma", "wave"),
     ("q4s", 64, 200, 1024, "rms", "wave"), ("q8h", 100, 1024, 512, "swiglu", "wave"),
@@ -267,3 +268,41 @@ def test_other_kernels_where_they_stay(ctx, aexq, orc):
         x = torch.zeros(16 * 1008, dtype=torch.float16, device="cuda")
         y = aexq.new_activation(16, 64, torch.float16, lay)
         ctx.plan_check(w, aexq.describe(x, 16, 1008), aexq.describe(y, 16, 64, lay), up=w)
+
+
+@pytest.mark.parametrize("fmt,m,n,k,epi,here", [
+    # long rows of few tiles, with the norm inside and without; groups of 16 sooner
+    ("q8h", 16, 1024, 12288, "plain", True), ("q8h", 16, 1024, 12416, "plain", False),
+    ("q8h", 16, 1024, 12416, "rms", True), ("q4g16s", 5, 64, 6272, "plain", False),
+    ("q4h", 5, 4200, 1152, "rms", False), ("q4h", 5, 4200, 1024, "rms", True),
+    # more than a workgroup per CU: pairs, streamed Q8, the norm over long rows
+    ("q8h", 7, 8190, 256, "swiglu", True), ("q8h", 7, 8200, 256, "swiglu", False),
+    ("q4h", 7, 8200, 256, "swiglu", True), ("q8h", 7, 16400, 256, "plain", False),
+    ("q4h", 7, 16400, 256, "plain", True), ("q4h", 9, 9000, 1664, "rms", False),
+    # exact pairs in groups of 16, on tiles of 32 rows by 32
+    ("q4g16s", 23, 8192, 1024, "swiglu", False), ("q4h", 23, 8192, 1024, "swiglu", True),
+    # tiles of 32 and 64 rows
+    ("q4h", 64, 4096, 6144, "plain", True), ("q4h", 64, 4096, 6272, "plain", False),
+    ("q8h", 43, 12672, 640, "plain", False), ("q8h", 43, 12160, 640, "plain", True),
+    ("q4h", 600, 2048, 1024, "plain", True), ("q4h", 600, 2048, 2176, "plain", False),
+    ("q4h", 600, 2048, 768, "plain", False),
+])
+def test_where_another_kernel_is_faster(ctx, aexq, fmt, m, n, k, epi, here):
+    """Both sides of the lines that the rule of the wave-split kernel draws
+    (planned only)."""
+    print(f"[gpu-case] wave split rule {fmt} m={m} n={n} k={k} {epi}", flush=True)
+    bits, group, f16, code = FORMATS[fmt]
+    sdt = np.float16 if f16 else np.float32
+    w = ctx.weight(aexq.QuantizedTensor(n * k, group or k, np.zeros(n * k * bits // 32, np.uint32),
+                                        np.ones(n * k // group if group else n, sdt), bits=bits,
+                                        nibble_code=code), n, k)
+    lay = aexq.LAYOUT_PACK4_LINEAR
+    x = torch.zeros(m * k, dtype=torch.float16, device="cuda")
+    y = aexq.new_activation(m, n, torch.float16, lay)
+    kw = {}
+    if epi in ("rms", "swiglu"):
+        kw.update(rmsnorm=True, rms_gamma=None, rms_eps=EPS)
+    if epi == "swiglu":
+        kw["up"] = w
+    plan = ctx.plan_check(w, aexq.describe(x, m, k), aexq.describe(y, m, n, lay), **kw)
+    assert (plan_kernel(plan) == "wave") == here, plan
