@@ -1093,21 +1093,32 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
       gc = QgemmConfig{fmt, bm, swiglu, sf16, g16, true, fd, k128};
       // eight waves on a tile, two along its rows, where the switches of the
       // four-wave forms are off
-      long long tiles = 0;  // of 128 x 128
+      long long ntiles = 0;  // of 128 weight rows
       for (int i = 0; i < count; ++i)
-        tiles += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + (swiglu ? 63 : 127)) /
-                 (swiglu ? 64 : 128) * w0->batch;
-      tiles *= (M + 127) / 128;
-      if (M > 64 && (fmt == kQ8 || fd) && !benv && !getenv("AEXQ_QGEMM_K64") && !getenv("AEXQ_SPLITK")) {
-        // From 96 tiles to one (Q4, whose codes each row half of the tile expands
-        // again) or two per CU (Q8), all resident at once and unsplit: the
+        ntiles += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + (swiglu ? 63 : 127)) /
+                  (swiglu ? 64 : 128) * w0->batch;
+      const int mtiles = (M + 127) / 128;
+      // the grid pads the weight tiles to eight: those of the last group add a
+      // column of row tiles to one XCD each (Q4, 1334 x 2304 x 512, 198 tiles in a
+      // grid of 264: 20.5 us against 13.9)
+      const long long g = (ntiles + 7) / 8 * 8 * mtiles, cu = ctx->cus;
+      if (M > 64 && (fmt == kQ8 || (fd && K % 128 == 0)) && !benv && !getenv("AEXQ_QGEMM_K64") &&
+          !getenv("AEXQ_SPLITK")) {
+        // From 96 tiles to one per CU, all resident at once and unsplit: the
         // four-wave tile leaves one wave a SIMD there, or splits K and pays the
         // partial planes (us, 1000 x 4096 x 4096: Q8 43 against 66, Q4-g16 47
-        // against 63; 512 x 8192 x 2048 Q8 26 against 30).  Past that its two
-        // workgroups a CU do as well with less expansion (2048 x 4096 x 1024 Q4 30
-        // against 37), and tiles of 256 weight rows were no faster (2048 x 8192
-        // pairs x 2048 Q8: 159 against 154 with half the bytes per product).
-        if (tiles >= 96 && tiles <= (fmt == kQ8 ? 2 : 1) * ctx->cus && (fmt == kQ8 || K % 128 == 0))
+        // against 63; 512 x 8192 x 2048 Q8 26 against 30).  Up to two per CU it
+        // still pays for Q8 (1413 x 2790 x 1920: 33 against 36), not for pairs
+        // (1154 x 2240 x 1920: 42 against 38) and not for Q4, whose codes each row
+        // half of the tile expands again (2048 x 4096 x 1024 37 against 30).
+        // Where the tiles leave CUs idle, long rows are better split (512 x 4096,
+        // 128 tiles, K = 8192: Q4 73 against 59, Q8 62 against 57), and one or two
+        // K steps of a single row tile run as well in four waves.  Tiles of 256
+        // weight rows were no faster (2048 x 8192 pairs x 2048 Q8: 159 against 154
+        // with half the bytes per product).
+        const int most = g <= cu * 3 / 4 ? (fmt == kQ8 ? (int)(16 * 256 * g / cu) : 2048)
+                         : g <= cu ? 16384 : (g <= 2 * cu && fmt == kQ8 && !swiglu ? 4096 : 0);
+        if (ntiles * mtiles >= cu * 3 / 8 && K <= most && (K > 256 || M > 96))
           gc = QgemmConfig{fmt, 128, swiglu, sf16, g16, true, fd, fmt == kQ4, 2};
       }
     }

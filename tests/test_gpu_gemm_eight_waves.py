@@ -116,3 +116,31 @@ def test_eight_wave_tiles(ctx, aexq, orc, bits, group, f16, m, n, k, epi, cols):
     elif epi == "bias":
         ref = 0.75 * (1.25 * bias[None].astype(np.float64) + ref)
     assert normwise(got, ref) <= (TOL32 if y32 else TOL), plan
+
+
+@pytest.mark.parametrize("fmt,m,n,k,pair,waves", [
+    # 96 tiles and one below; grids padded to eight weight tiles past one per CU
+    ((8, 0), 1000, 1536, 1024, False, 8), ((8, 0), 1000, 1408, 1088, False, 4),
+    ((4, 32), 1334, 2304, 512, False, 4), ((4, 32), 1334, 2048, 512, False, 8),
+    # one and two tiles per CU, weights and pairs
+    ((8, 0), 2048, 4096, 1024, False, 8), ((8, 0), 2100, 4096, 1024, False, 4),
+    ((4, 16), 2048, 2048, 1024, False, 8), ((4, 16), 2048, 2176, 1024, False, 4),
+    ((8, 0), 2048, 1024, 1024, True, 8), ((8, 0), 2048, 1088, 1024, True, 4),
+    # long rows on idle CUs; a step or two of one row tile
+    ((8, 0), 512, 4096, 2048, False, 8), ((8, 0), 512, 4096, 2112, False, 4),
+    ((4, 32), 512, 4096, 2048, False, 8), ((4, 32), 512, 4096, 2176, False, 4),
+    ((8, 0), 1024, 4096, 8192, False, 8), ((4, 32), 90, 13312, 256, False, 4),
+])
+def test_where_eight_waves_are_taken(ctx, aexq, monkeypatch, no_wave, fmt, m, n, k, pair, waves):
+    """Both sides of the lines of the rule (planned only)."""
+    print(f"[gpu-case] eight waves rule {fmt} m={m} n={n} k={k} pair={pair}", flush=True)
+    bits, group = fmt
+    w = ctx.weight(aexq.QuantizedTensor(n * k, group or k, np.zeros(n * k * bits // 32, np.uint32),
+                                        np.ones(n * k // group if group else n, np.float16),
+                                        bits=bits), n, k)
+    x = torch.zeros(m * k, dtype=torch.float16, device="cuda")
+    lay = aexq.LAYOUT_PACK4_LINEAR
+    y = aexq.new_activation(m, n, torch.float16, lay)
+    plan = ctx.plan_check(w, aexq.describe(x, m, k), aexq.describe(y, m, n, lay),
+                          **({"up": w} if pair else {}))
+    assert plan.split()[0] == "kernel=qgemm" and f" waves={waves} " in plan, plan
