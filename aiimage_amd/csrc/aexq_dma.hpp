@@ -25,7 +25,7 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // barrier for the other waves' -- and the memory clobber keeps the compiler
 // from moving LDS accesses across a load.
 template <int BYTES>
-__device__ __forceinline__ void dma(__amdgpu_buffer_rsrc_t r, uint32_t lds, int voff) {
+__device__ __forceinline__ void dma(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t voff) {
   static_assert(BYTES == 16 || BYTES == 4, "dword or dwordx4");
   if constexpr (BYTES == 16)
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"

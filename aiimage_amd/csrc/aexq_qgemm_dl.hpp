@@ -134,11 +134,17 @@ struct QGemmDL {
       return ((r >> 1) & 3) + 8 * ((r >> 3) & 1);
   }
 
+  // Byte offsets are unsigned, as the hardware takes them: kNoLoad is past every
+  // resource, and stays there when a step past the end adds it once more.
+  static constexpr uint32_t kNoLoad = 1u << 30;
+  static __device__ __host__ constexpr uint32_t past_end(bool live) { return live ? 0 : kNoLoad; }
+  static_assert(kNoLoad + past_end(false) > kNoLoad, "an offset past the end wraps around");
+
   struct Src {
     __amdgpu_buffer_rsrc_t xr, wr, sr;
-    int oa[A_INST];  // per-lane byte offsets of step 0
-    int ob[B_INST];
-    int os[S_INST > 0 ? S_INST : 1];
+    uint32_t oa[A_INST];  // per-lane byte offsets of step 0
+    uint32_t ob[B_INST];
+    uint32_t os[S_INST > 0 ? S_INST : 1];
   };
 
   static __device__ __forceinline__ Src source(const QmvParams& p, const QmvMat& mt, int b,
@@ -211,7 +217,7 @@ struct QGemmDL {
         const int byte = 256 * j + 4 * lane;  // in the step's scale block [row][SPR]
         const int srow = byte / (SPR * SB), sin = byte % (SPR * SB);
         const int wrow = PAIR ? (srow & (HB - 1)) : srow;
-        s.os[i] = 256 * j >= S_BYTES ? (1 << 30) : wrow * p.groups_per_row * SB + sin;
+        s.os[i] = 256 * j >= S_BYTES ? kNoLoad : wrow * p.groups_per_row * SB + sin;
       }
     }
     return s;
@@ -221,7 +227,7 @@ struct QGemmDL {
   // same loads past the resources (zeros, no traffic).
   static __device__ __forceinline__ void issue(const Src& s, uint32_t base, int wave, int st,
                                                bool live = true) {
-    const int dead = live ? 0 : 1 << 30;
+    const uint32_t dead = past_end(live);
 #pragma unroll
     for (int t = 0; t < A_INST; ++t)
       dma<16>(s.xr, base + (wave * A_INST + t) * 1024, s.oa[t] + (st * RA + dead));
