@@ -1161,6 +1161,11 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
     if (!qmmk_pick(shape, &kc.mt, &kc.nt, &kc.waves)) return;
     const char* env = getenv("AEXQ_QMMK_TILE");  // tuning: "mt:nt:waves"
     if (env && sscanf(env, "%d:%d:%d", &kc.mt, &kc.nt, &kc.waves) != 3) return;
+    // (the generic kernel spreads its rows over two grid dimensions; a dimension
+    // holds 2^32 - 1 threads)
+    const long long blocks = ((t16 + kc.nt - 1) / kc.nt + count + 7) / 8 * 8 *
+                             ((M + 16LL * kc.mt - 1) / (16 * kc.mt));
+    if (blocks * 64 * kc.waves > 0xffffffffLL) return;
     const QmmkEntry* e = qmmk_find(kc);
     if (!e) return;
     plan->kentry = e;

@@ -243,6 +243,21 @@ def test_rows_too_far_apart_for_its_offsets(ctx, aexq, orc):
     assert kernel(k, 1 << 22) != "kernel=wave"
 
 
+@pytest.mark.parametrize("m,kernel", [(1 << 19, "wave"), (1 << 20, "generic")])
+def test_more_rows_than_one_grid_dimension_holds(ctx, aexq, m, kernel):
+    """Ragged launches of 2^32 threads and more stay on the generic kernel, whose
+    rows have a grid dimension of their own (planned only: no such rows are there)."""
+    print(f"[gpu-case] wave split grid m={m}", flush=True)
+    n, k = 16400, 48
+    w = ctx.weight(aexq.QuantizedTensor(n * k, k, np.zeros(n * k // 4, np.uint32),
+                                        np.ones(n, np.float16), bits=8), n, k)
+    x = aexq.describe(torch.zeros(k, dtype=torch.float16, device="cuda"), 1, k)
+    y = aexq.describe(torch.zeros(n, dtype=torch.float16, device="cuda"), 1, n)
+    for d in (x, y):
+        d.logical.h = d.storage.h = m
+    assert plan_kernel(ctx.plan_check(w, x, y)) == kernel
+
+
 def test_other_kernels_where_they_stay(ctx, aexq, orc):
     """Forms the wave-split kernel does not take: one row and short ragged rows
     stream, K of odd 64s is tiled, fp32 rows and other groups go where they went."""
