@@ -1131,11 +1131,12 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
   // launches with few output tiles: K split over a workgroup's waves
   // (aexq_qmmk.hpp).  K % 128 == 0: M >= 2; up to 32 rows Q4 products stay
   // exact and RMSNorm-in runs inside the kernel, above that Q4 weight tiles are
-  // fp16 and the norm is the row pre-pass, as in the tiled GEMM.  Any other K
-  // (rows past 8, or rows whose codes the streaming kernel cannot chunk): where
-  // only the generic kernel would be left (77 x 1008 x 1001: 5.7 us against
-  // 54.5); exact products.  The AEXQ_* switches that name another kernel's form
-  // keep that kernel.
+  // fp16 and the norm is the row pre-pass, as in the tiled GEMM.  K that is no
+  // multiple of 64 (rows past 8, or rows whose codes the streaming kernel cannot
+  // chunk): where only the generic kernel would be left (77 x 1008 x 1001: 5.7
+  // us against 54.5); exact products.  K of odd 64s keeps the kernels that it
+  // has (split K, the tiled GEMM): the ragged form is not compared with those.
+  // The AEXQ_* switches that name another kernel's form keep that kernel.
   auto try_wave = [&]() {
     const bool rag = K % 128 != 0;
     const int unit = fmt == kQ4 && w0->block == 32 ? 32 : 16;

@@ -110,9 +110,11 @@ hipError_t rope_kv_launch(void* q, const void* k, const void* v, void* kcache, v
 //   M = max m_s, L = sum l_s e^(m_s - M), out = sum acc_s e^(m_s - M) / max(L, 1e-20).
 // That merge reads splits x G rows of 528 bytes through one CU, so a long cache
 // takes longer splits rather than more of them (attn_splits): with 64 positions
-// a split, 16 heads over 4 x 16384 positions took 21.0 us, half of them in the
-// merge, now 13.1 (32 MB: 5 us at the rate the shared cache level gives); up to
-// 64 positions there is one split and nothing to merge (7.4 -> 5.0 us).
+// a split, 16 heads over 4 x 16384 positions (32 MB) took 21.0 us, half of them
+// in the merge, now 12.5 with the rows in the last-level cache (5 us at the rate
+// that gives); on caches in turn, whose rows come from HBM, 22.5 -> 13.3; the
+// first pass over rows just written, 62 -> 51.  Up to 64 positions there is one
+// split and nothing to merge (7.4 -> 5.0 us).
 // head_dim == 128.
 // ---------------------------------------------------------------------------
 constexpr int kAttnDim = 128;

@@ -268,9 +268,10 @@ int attn_most_splits(int len);
 int attn_max_len();
 int attn_part_stride();  // fp32 words per (head, split) partial row
 int attn_counter_stride();  // ints between the kv heads' split counters
-// part: hq * splits * (128 + 2) floats; counters: hkv ints, zero before the
-// first launch (every launch leaves them zero).  knew/vnew/cosv/sinv non-null:
-// RoPE of q and of the new k row plus the K/V append at position len - 1.
+// part: hq * splits rows of attn_part_stride() floats; counters: one int every
+// attn_counter_stride() per kv head, zero before the first launch (every launch
+// leaves them zero).  knew/vnew/cosv/sinv non-null: RoPE of q and of the new k row
+// plus the K/V append at position len - 1.
 // posp non-null: the position is *posp (clamped to the capacity), read on the
 // device, the grid is sized for `cap` positions and cosv/sinv are [cap][64]
 // tables whose row *posp is used; `len` is ignored.

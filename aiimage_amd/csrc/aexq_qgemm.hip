@@ -64,8 +64,8 @@ int qgemm_rows_per_tile(bool pair) { return pair ? 64 : 128; }
 
 int qgemm_blocks_per_cu(const QgemmEntry* e) {
   static int cache[kCountG] = {0};
+  if (e->cfg.wm != 1) return 1;  // (for split K, which the eight-wave tiles do not take)
   const int idx = (int)(e - kTableG);
-  if (idx < 0 || idx >= kCountG) return 1;  // the eight-wave tiles fill a CU's LDS
   if (cache[idx] == 0) {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, e->fn, kThreads, 0) != hipSuccess || n < 1)

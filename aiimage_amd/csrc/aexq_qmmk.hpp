@@ -1,6 +1,6 @@
 // Quantized matmul for launches with few output tiles (one layer's linears at
-// M = 2..128): Y[M][N] = X[M][K] W[N][K]^T, the K of a tile split over the
-// waves of one workgroup.
+// M = 2 to some hundreds; K that is no multiple of 64 at any M): Y[M][N] =
+// X[M][K] W[N][K]^T, the K of a tile split over the waves of one workgroup.
 //
 // A workgroup owns 16 MT activation rows by 16 NT weight rows (a SwiGLU pair:
 // the same rows of both weights) and the whole of K, so nothing is left for a
@@ -9,15 +9,20 @@
 // of dependent round trips, so a wave asks for as many of its slices as its
 // share of LDS holds at once (LDS-direct loads into a ring of `depth` slots of
 // its own, which needs no barrier: a wave waits for its own loads only), and
-// the residual and the Q8 row scales are requested at the start.
+// the residual and the Q8 row scales are requested at the start.  With one
+// workgroup per CU that is up to four slices; launches of more, whose rings
+// share a CU, hold one slice a wave on 32 x 32 and 64 x 32 tiles (a slot of all
+// waves takes 42 to 80 KB), and there only the other workgroups of the CU cover
+// the wait for the next.
 //
 // The loads go through LDS rather than straight into fragments because of how
 // a CU fetches: consecutive lanes reading 16 consecutive bytes of one row keep
 // to one cache line, while MFMA lanes (row l % 16, lane group l / 16) would
-// touch 16 lines per instruction, which ran at 20 bytes per clock and CU.
-// Slots hold rows with their 16-byte chunks XOR-swizzled so that the fragment
-// reads meet no bank conflicts (gfx950 serves 32 lanes' 16-byte reads per pass
-// over 512 bytes).
+// touch 16 lines per instruction (measured below).  Slots hold rows with their
+// 16-byte chunks XOR-swizzled against bank conflicts in the fragment reads.
+// That does not take them all: SQ_LDS_BANK_CONFLICT counts 2.3 (Q4) to 3.4 (Q8)
+// stall cycles per LDS instruction, 1.1 to 1.5 with RMSNorm-in.  The MFMA units
+// are busy 0.4 to 2.7% of the time on 16-row tiles, 2.7 to 11.5% on larger ones.
 //
 // Which K the lane groups g of an MFMA carry:
 //  * Q8: of each 64-code half codes 16 g .. 16 g + 15, eight to each of its
@@ -521,5 +526,13 @@ __global__ __launch_bounds__(64 * W) void qmmk_kernel(const QmvParams p, int mti
     }
   }
 }
+
+// An entry of a table of instantiations.
+#define QMMK_ENTRY(FMT, G, SF16, FD, MT, NT, W, PAIR, RMS, RAG)          \
+  QmmkEntry {                                                           \
+    QmmkConfig{FMT, G, SF16, FD, MT, NT, W, PAIR, RMS, RAG},             \
+        &qmmk_kernel<FMT, G, SF16, FD, MT, NT, W, PAIR, RMS, RAG>,       \
+        QmmK<FMT, G, SF16, FD, MT, NT, PAIR, RMS, RAG>::SLOT             \
+  }
 
 }  // namespace aexq

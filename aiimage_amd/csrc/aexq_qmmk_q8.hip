@@ -3,12 +3,7 @@
 
 namespace aexq {
 
-#define QMMK(G, SF16, MT, NT, W, PAIR, RMS, RAG)                              \
-  QmmkEntry {                                                                \
-    QmmkConfig{kQ8, G, SF16, false, MT, NT, W, PAIR, RMS, RAG},               \
-        &qmmk_kernel<kQ8, G, SF16, false, MT, NT, W, PAIR, RMS, RAG>,         \
-        QmmK<kQ8, G, SF16, false, MT, NT, PAIR, RMS, RAG>::SLOT               \
-  }
+#define QMMK(G, SF16, ...) QMMK_ENTRY(kQ8, G, SF16, false, __VA_ARGS__)
 #define QMMK_ALL(G, SF16)                                                                          \
   QMMK(G, SF16, 1, 1, 8, false, false, false), QMMK(G, SF16, 1, 2, 8, false, false, false),       \
       QMMK(G, SF16, 2, 1, 8, false, false, false), QMMK(G, SF16, 2, 2, 8, false, false, false),   \
