@@ -1112,11 +1112,12 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
         // (1154 x 2240 x 1920: 42 against 38) and not for Q4, whose codes each row
         // half of the tile expands again (2048 x 4096 x 1024 37 against 30).
         // Where the tiles leave CUs idle, long rows are better split (512 x 4096,
-        // 128 tiles, K = 8192: Q4 73 against 59, Q8 62 against 57), and one or two
-        // K steps of a single row tile run as well in four waves.  Tiles of 256
+        // 128 tiles, K = 8192: Q4 73 against 59, Q8 62 against 57; stacked copies,
+        // whose rows fewer tiles share, sooner: 16 of 242 x 348 x 2048 40 against
+        // 33), and one or two K steps of a single row tile run as well in four waves.  Tiles of 256
         // weight rows were no faster (2048 x 8192 pairs x 2048 Q8: 159 against 154
         // with half the bytes per product).
-        const int most = g <= cu * 3 / 4 ? (fmt == kQ8 ? (int)(16 * 256 * g / cu) : 2048)
+        const int most = g <= cu * 3 / 4 ? (fmt == kQ8 ? (int)(16 * 256 * g / cu) : w0->batch > 1 ? 1024 : 2048)
                          : g <= cu ? 16384 : (g <= 2 * cu && fmt == kQ8 && !swiglu ? 4096 : 0);
         if (ntiles * mtiles >= cu * 3 / 8 && K <= most && (K > 256 || M > 96))
           gc = QgemmConfig{fmt, 128, swiglu, sf16, g16, true, fd, fmt == kQ4, 2};
@@ -1153,18 +1154,21 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
     const bool fused = rms_in && (rag || M <= 32) && getenv("AEXQ_RMS_PREPASS") == nullptr;
     // (the kernel reads gamma[0 .. K) of fp16 rows)
     if (fused ? !(rms_ok && x_ok) : !x_ok && !rms_in) return;
-    long long t16 = 0;
-    for (int i = 0; i < count; ++i)
-      t16 += (long long)((ys[i] ? yv[i].padded : ws[i]->n) + 15) / 16 * w0->batch;
+    long long t16 = 0, t32 = 0;
+    for (int i = 0; i < count; ++i) {
+      const int n = ys[i] ? yv[i].padded : ws[i]->n;
+      t16 += (n + 15LL) / 16 * w0->batch;
+      t32 += (n + 31LL) / 32 * w0->batch;
+    }
     QmmkConfig kc{fmt, fmt == kQ8 ? 0 : w0->block, w0->scale_dtype == AEXQ_DTYPE_F16,
                   !rag && M > 32 && fd, 1, 1, 8, swiglu, fused, rag};
-    const QmmkShape shape{M, K, t16, fmt, kc.g, kc.fd, swiglu, fused, rag, ctx->cus};
+    const QmmkShape shape{M, K, t16, t32, fmt, kc.g, kc.fd, swiglu, fused, rag, ctx->cus};
     if (!qmmk_pick(shape, &kc.mt, &kc.nt, &kc.waves)) return;
     const char* env = getenv("AEXQ_QMMK_TILE");  // tuning: "mt:nt:waves"
     if (env && sscanf(env, "%d:%d:%d", &kc.mt, &kc.nt, &kc.waves) != 3) return;
     // (the generic kernel spreads its rows over two grid dimensions; a dimension
     // holds 2^32 - 1 threads)
-    const long long blocks = ((t16 + kc.nt - 1) / kc.nt + count + 7) / 8 * 8 *
+    const long long blocks = ((kc.nt == 1 ? t16 : t32) + 7) / 8 * 8 *
                              ((M + 16LL * kc.mt - 1) / (16 * kc.mt));
     if (blocks * 64 * kc.waves > 0xffffffffLL) return;
     const QmmkEntry* e = qmmk_find(kc);

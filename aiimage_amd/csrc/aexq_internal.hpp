@@ -202,11 +202,11 @@ const QmmkEntry* qmmk_table_q8(int* count);
 const QmmkEntry* qmmk_table_q4(int* count);     // exact products
 const QmmkEntry* qmmk_table_q4_fd(int* count);  // fp16 weight tiles
 const QmmkEntry* qmmk_find(const QmmkConfig& cfg);
-// A launch of the wave-split matmul: m rows by t16 16-row weight blocks (over
-// every matrix and copy), K long, on a part of `cus` CUs.
+// A launch of the wave-split matmul: m rows by t16 tiles of 16 or t32 of 32
+// weight rows (over every matrix and copy), K long, on a part of `cus` CUs.
 struct QmmkShape {
   int m, k;
-  long long t16;
+  long long t16, t32;
   int fmt, g;
   bool fd, pair, rms, rag;  // as in QmmkConfig
   int cus;

@@ -20,9 +20,9 @@
 // to one cache line, while MFMA lanes (row l % 16, lane group l / 16) would
 // touch 16 lines per instruction (measured below).  Slots hold rows with their
 // 16-byte chunks XOR-swizzled against bank conflicts in the fragment reads.
-// That does not take them all: SQ_LDS_BANK_CONFLICT counts 2.3 (Q4) to 3.4 (Q8)
-// stall cycles per LDS instruction, 1.1 to 1.5 with RMSNorm-in.  The MFMA units
-// are busy 0.4 to 2.7% of the time on 16-row tiles, 2.7 to 11.5% on larger ones.
+// That does not take them all: SQ_LDS_BANK_CONFLICT counts 1.0 to 4.2 stall cycles
+// per LDS instruction over a layer's linears.  The MFMA units are busy 0.5 to 2.4%
+// of the time on 16-row tiles, 2.2 to 10.5% on larger ones.
 //
 // Which K the lane groups g of an MFMA carry:
 //  * Q8: of each 64-code half codes 16 g .. 16 g + 15, eight to each of its

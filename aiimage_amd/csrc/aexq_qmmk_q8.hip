@@ -45,15 +45,16 @@ static constexpr int kRingLds = 152 * 1024;
 // tiles to one XCD); limits on K are there because a workgroup walks all of it
 // while the other kernels split it over more of them.  The lines are drawn where
 // 55 thousand random launches (M 2..2048, N 32..40000, K 128..32768, rotated
-// weights, each against the kernel that it takes with this one off) turn; of 21
-// thousand others that they let through, 16 are more than 3% slower and 84% more
-// than 20% faster.  Both sides of the lines, us, here / there:
+// weights, each against the kernel that it takes with this one off) turn; of 36
+// thousand others that they let through, stacked copies and groups among them, 20
+// are more than 3% slower and five in six more than 20% faster.  Both sides of the
+// lines, us, here / there:
 bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
   const int m = q.m, K = q.k;
   const bool q8 = q.fmt == kQ8, g16 = q.g == 16, pair = q.pair;
   const bool exact = q.fmt == kQ4 && !q.fd;
   const long long m16 = (m + 15) / 16, m32 = (m + 31) / 32, m64 = (m + 63) / 64;
-  const long long t16 = q.t16, t32 = (t16 + 1) / 2;
+  const long long t16 = q.t16, t32 = q.t32;
   const long long cu = q.cus;
   auto take = [&](int a, int b, int w) {
     *mt = a;
@@ -62,8 +63,10 @@ bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
     return true;
   };
   // workgroups of tiles of 16 nt weight rows, as the grid pads them
-  auto grid = [&](int nt_, long long mtiles) { return ((t16 + nt_ - 1) / nt_ + 7) / 8 * 8 * mtiles; };
-  // ragged K: no other matrix-core kernel takes it
+  auto grid = [&](int nt_, long long mtiles) { return ((nt_ == 1 ? t16 : t32) + 7) / 8 * 8 * mtiles; };
+  // ragged K: no other matrix-core kernel takes it, and one row of less than half
+  // a slice is all launch (N = 97, K = 48: 4.4 / 3.9)
+  if (q.rag && m == 1 && K < 64) return false;
   if (q.rag) return t16 * m16 <= cu * 5 / 4 ? take(1, 1, 8) : take(2, 2, 4);
   if (m <= 32) {
     if (t16 * m16 <= cu * 5 / 4) {
@@ -87,7 +90,7 @@ bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
       // 256, M = 7: 10.6 / 6.4; groups of 32, whose other kernel is slower, 7.6 / 8.3)
       if (pair) return !q8 && !g16 && g <= 2 * cu && K <= 1024 && take(1, 2, 8);
       // the norm reads rows longer than the ring twice
-      if (q.rms) return g <= 2 * cu && K <= 1536 && take(1, 2, 8);
+      if (q.rms) return g <= 2 * cu && K <= 1024 && take(1, 2, 8);
       // past two per CU the launch streams from HBM, which persistent workgroups
       // do better (Q8, N = 26496, K = 256, M = 7: 8.3 / 6.1), but for groups of 32
       // (N = 24150, K = 128: 5.2 / 6.4)
@@ -112,7 +115,7 @@ bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
   // 1024: 18.8 us against 21.1)
   if (q8 && m > 64 && (t16 + (pair ? 3 : 7)) / (pair ? 4 : 8) * ((m + 127) / 128) >= cu * 3 / 8) return false;
   if (!pair && t16 * m16 <= cu * 5 / 2)  // 1024 x 2048, M = 128: 6.7 us; 2:2 7.2
-    return (grid(1, m32) <= cu || K <= 6144) && take(2, 1, 8);
+    return K <= (grid(1, m32) <= cu ? 24576 : 6144) && take(2, 1, 8);
   if (t32 * m32 <= cu)  // 4096 x 4096, M = 64: 9.9 us; 4 waves 10.9; K = 28672: 48 / 39
     return !(exact && pair && g16) && K <= (pair ? 4096 : 6144) && take(2, 2, 8);
   if (t32 * m32 <= cu * 7 / 2) {
@@ -132,9 +135,12 @@ bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
   }
   // larger tiles fetch less per product (2459 x 1024, M = 556: 14.9 / 24.8); short
   // rows leave their four waves a slice or two each (N = 2816, K = 768, M = 398:
-  // 14.1 / 13.1), long ones wait for them (N = 993, K = 3840, M = 1499: 54 / 40)
+  // 14.1 / 13.1), long ones wait for them (N = 993, K = 3840, M = 1499: 54 / 40),
+  // and a single row of tiles is the tiled GEMM's sooner (Q8, N = 24030, K = 1280,
+  // M = 45: 19.1 / 14.0)
   const long long g = grid(2, m64);
-  return !pair && !exact && g <= 3 * cu && K >= 896 && K <= (g <= cu * 5 / 2 ? 2048 : 1280) && take(4, 2, 4);
+  return !pair && !exact && g <= (m > 64 ? 3 : 2) * cu && K >= 896 &&
+         K <= (g <= cu * 5 / 2 ? 2048 : 1280) && take(4, 2, 4);
 }
 
 int qmmk_depth(const QmmkEntry* e, int k, long long wgs, int cus) {

@@ -300,24 +300,32 @@ def test_other_kernels_where_they_stay(ctx, aexq, orc):
     ("q4h", 64, 4096, 6144, "plain", True), ("q4h", 64, 4096, 6272, "plain", False),
     ("q8h", 43, 12672, 640, "plain", False), ("q8h", 43, 12160, 640, "plain", True),
     ("q4h", 600, 2048, 1024, "plain", True), ("q4h", 600, 2048, 2176, "plain", False),
-    ("q4h", 600, 2048, 768, "plain", False),
+    ("q4h", 600, 2048, 768, "plain", False), ("q8h", 45, 24030, 1280, "plain", False),
+    # stacked copies, whose odd block fills a tile of its own
+    ("q8h", 7, (22, 352), 256, "swiglu", True), ("q8h", 7, (22, 358), 256, "swiglu", False),
+    # ragged rows of less than half a slice
+    ("q4g16s", 1, 97, 48, "plain", False), ("q4g16s", 1, 97, 80, "plain", True),
 ])
 def test_where_another_kernel_is_faster(ctx, aexq, fmt, m, n, k, epi, here):
     """Both sides of the lines that the rule of the wave-split kernel draws
     (planned only)."""
     print(f"[gpu-case] wave split rule {fmt} m={m} n={n} k={k} {epi}", flush=True)
     bits, group, f16, code = FORMATS[fmt]
+    copies, n = n if isinstance(n, tuple) else (1, n)
     sdt = np.float16 if f16 else np.float32
     w = ctx.weight(aexq.QuantizedTensor(n * k, group or k, np.zeros(n * k * bits // 32, np.uint32),
                                         np.ones(n * k // group if group else n, sdt), bits=bits,
                                         nibble_code=code), n, k)
+    if copies > 1:
+        w = w.replicate(copies)
     lay = aexq.LAYOUT_PACK4_LINEAR
     x = torch.zeros(m * k, dtype=torch.float16, device="cuda")
-    y = aexq.new_activation(m, n, torch.float16, lay)
+    y = aexq.new_activation(m, n, torch.float16, lay, batch=copies)
+    yd = aexq.describe(y, m, n, lay, batch=copies, batch_stride=y.numel() // copies)
     kw = {}
     if epi in ("rms", "swiglu"):
         kw.update(rmsnorm=True, rms_gamma=None, rms_eps=EPS)
     if epi == "swiglu":
         kw["up"] = w
-    plan = ctx.plan_check(w, aexq.describe(x, m, k), aexq.describe(y, m, n, lay), **kw)
+    plan = ctx.plan_check(w, aexq.describe(x, m, k), yd, **kw)
     assert (plan_kernel(plan) == "wave") == here, plan
