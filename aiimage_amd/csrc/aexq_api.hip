@@ -1114,11 +1114,14 @@ static aexq_status make_plan(aexq_ctx* ctx, int count, const aexq_weight* const*
         // Where the tiles leave CUs idle, long rows are better split (512 x 4096,
         // 128 tiles, K = 8192: Q4 73 against 59, Q8 62 against 57; stacked copies,
         // whose rows fewer tiles share, sooner: 16 of 242 x 348 x 2048 40 against
-        // 33), and one or two K steps of a single row tile run as well in four waves.  Tiles of 256
-        // weight rows were no faster (2048 x 8192 pairs x 2048 Q8: 159 against 154
-        // with half the bytes per product).
-        const int most = g <= cu * 3 / 4 ? (fmt == kQ8 ? (int)(16 * 256 * g / cu) : w0->batch > 1 ? 1024 : 2048)
-                         : g <= cu ? 16384 : (g <= 2 * cu && fmt == kQ8 && !swiglu ? 4096 : 0);
+        // 33), and one or two K steps of a single row tile run as well in four
+        // waves.  Tiles of 256 weight rows were no faster (2048 x 8192 pairs x 2048
+        // Q8: 159 against 154 with half the bytes per product).
+        int most = 16384;
+        if (g <= cu * 3 / 4)
+          most = fmt == kQ8 ? (int)(16 * 256 * g / cu) : (w0->batch > 1 ? 1024 : 2048);
+        else if (g > cu)
+          most = g <= 2 * cu && fmt == kQ8 && !swiglu ? 4096 : 0;
         if (ntiles * mtiles >= cu * 3 / 8 && K <= most && (K > 256 || M > 96))
           gc = QgemmConfig{fmt, 128, swiglu, sf16, g16, true, fd, fmt == kQ4, 2};
       }

@@ -113,7 +113,8 @@ bool qmmk_pick(const QmmkShape& q, int* mt, int* nt, int* waves) {
     return (grid(1, m16) <= cu || K <= 6144) && take(1, 1, 8);
   // Q8 from 96 tiles of 128 x 128: the tiled GEMM's eight-wave form (512 x 3072 x
   // 1024: 18.8 us against 21.1)
-  if (q8 && m > 64 && (t16 + (pair ? 3 : 7)) / (pair ? 4 : 8) * ((m + 127) / 128) >= cu * 3 / 8) return false;
+  if (q8 && m > 64 && (t16 + (pair ? 3 : 7)) / (pair ? 4 : 8) * ((m + 127) / 128) >= cu * 3 / 8)
+    return false;
   if (!pair && t16 * m16 <= cu * 5 / 2)  // 1024 x 2048, M = 128: 6.7 us; 2:2 7.2
     return K <= (grid(1, m32) <= cu ? 24576 : 6144) && take(2, 1, 8);
   if (t32 * m32 <= cu)  // 4096 x 4096, M = 64: 9.9 us; 4 waves 10.9; K = 28672: 48 / 39

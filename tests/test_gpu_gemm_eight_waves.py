@@ -1,6 +1,7 @@
-"""The eight-wave tiles of the LDS-direct GEMM against the float64 oracle: one K step to more than the ring holds, tails of
-one and two steps, ragged rows and columns, pairs, residual, bias and
-head-packed outputs, every scale format.
+"""The eight-wave tiles of the LDS-direct GEMM against the float64 oracle: one K
+step to more than the ring holds, tails of one and two steps, ragged rows and
+columns, pairs, residual, bias and head-packed outputs, every scale format; and
+the rule that chooses them.
 
 Bars as in the other GEMM tests: 1e-5 of the largest value for plain fp32
 outputs against the weights the plan multiplies, 1e-3 for fp16."""
